@@ -1,6 +1,7 @@
 // SwiGLU grouped GEMM for the PlaceMoE expert layer on gfx950.
 //
-// One persistent kernel template serves every GEMM of the layer:
+// Persistent kernels (one block or more per CU) serve every GEMM of the layer;
+// calls whose copies hold few rows go to few_rows.h:
 //   KIND_FC1   X[a] @ [Wgate;Wup][g]^T with the SwiGLU forward epilogue
 //   KIND_NT    A[a] @ B[g]^T                       (fc2 forward)
 //   KIND_NN    A[a] @ B[g]                         (fc1 dgrad)
@@ -127,7 +128,7 @@ struct GemmParams {
   RowSrc a, b;
   const int32_t* offsets;
   int32_t G;
-  int64_t M, N, K;  // ragged-M kinds: N, K used.  KIND_TN: M, N, and K = rows of A and B.
+  int64_t M, N, K;  // ragged-M kinds: M = rows over all groups.  KIND_TN: M, N, and K = rows of A and B.
   int64_t I;        // SwiGLU width for KIND_FC1 and KIND_NNS
   bf16_t* c0;
   bf16_t* c1;
@@ -2145,6 +2146,8 @@ __global__ __launch_bounds__(NT, 1) void grouped_gemm_w4_kernel(GemmParams P) {
 
 }  // namespace w4
 
+#include "few_rows.h"
+
 // Buffer offsets are 32-bit: one descriptor covers at most 2 GiB.
 bool fits_rsrc(int64_t rows, int64_t ld) { return rows * ld * 2 < (int64_t)0x7fffffff; }
 
@@ -2187,6 +2190,37 @@ constexpr int64_t kRsMaxRowsPerCopy = 8 * kBM;
 template <int KIND>
 constexpr bool use_w4() { return PMX_GEMM_W4 && ((PMX_W4_KINDS >> KIND) & 1); }
 
+// Copies with few rows (few_rows.h).  The host knows the average rows per copy,
+// M / G, not the counts.  Up to kFewRows64 rows on average 64 x 256 tiles, up
+// to kFewRows128 128 x 256 tiles, beyond that the kernels above, whose
+// 256-row tiles read each weight strip for twice the rows.  Where the lines
+// lie (us; 64-row / 128-row tiles / 256-row kernels; 128 or 160 copies of the
+// 2048 x 768 layer, row counts log-normal with sigma 0.5):
+//   rows    fc1             fc2             fc2 dgrad       fc1 dgrad
+//   4.8     177 / 178 / 267  90 /  92 / 108  90 /  92 / 140 169 / 171 / 204
+//   25      187 / 191 / 267 107 /  99 / 105 108 / 110 / 145 194 / 184 / 196
+//   96      223 / 211 / 268 119 / 116 / 109 130 / 119 / 144 199 / 196 / 196
+//   150     266 / 227 / 270 156 / 129 / 115 178 / 160 / 152 252 / 216 / 210
+//   256     366 / 300 / 328 228 / 181 / 148 240 / 207 / 221 360 / 288 / 267
+// fc1 and the fc2 dgrad run on the four-wave kernel, whose loads have one
+// K-tile to land, and gain the most; fc2 and the fc1 dgrad on the
+// register-staged kernel (two K-tiles).  PMX_FEW_ROWS=0 builds without it (the
+// test variants of the 256-row kernels).
+#ifndef PMX_FEW_ROWS
+#define PMX_FEW_ROWS 1
+#endif
+using Few64 = fr::Cfg<1, 8, 4, 2, 2, 3, 1>;   // 64 x 256 tiles, 40 KB stages
+using Few128 = fr::Cfg<2, 4, 4, 4, 2, 3, 1>;  // 128 x 256 tiles, 48 KB stages
+constexpr int64_t kFewRows64[4] = {40, 16, 16, 40};     // fc1, fc2, fc1 dgrad, fc2 dgrad
+constexpr int64_t kFewRows128[4] = {224, 48, 64, 120};
+
+template <int KIND, class CF>
+int launch_few(const GemmParams& P, int cus, hipStream_t stream) {
+  fr::few_rows_grouped_gemm_kernel<KIND, CF><<<cus * CF::BPC, CF::NT, 0, stream>>>(P);
+  PMX_LAUNCH_CHECK();
+  return PMX_OK;
+}
+
 template <int KIND>
 int launch(const GemmParams& P, hipStream_t stream) {
   // The LDS tile table keeps an n-tile index in 19 bits.
@@ -2219,6 +2253,10 @@ int launch(const GemmParams& P, hipStream_t stream) {
       grouped_gemm_kernel<KIND_TN, kBM><<<grid, NTHREADS, 0, stream>>>(P);
     }
   } else {
+    // Weights in two tensors: the few-rows kernel picks one per K-tile.
+    const bool few = PMX_FEW_ROWS && P.G <= fr::kMaxG && (KIND != KIND_NN || P.b.split >= P.K || P.b.split % BK == 0);
+    if (few && P.M <= kFewRows64[KIND] * P.G) return launch_few<KIND, Few64>(P, grid, stream);
+    if (few && P.M <= kFewRows128[KIND] * P.G) return launch_few<KIND, Few128>(P, grid, stream);
     // FAST: K a multiple of 64, dgrad weights not split (P.b.split >= K).
     // RS (register-staged operands): fc1 and fc2 always; the fc1 dgrad when
     // the copies are small (under 8 m-tiles of rows on average), where each
@@ -2284,6 +2322,7 @@ int PMX_GEMM_FN(pmx_gemm_fc1_swiglu_fwd)(const void* X, const void* w_gate, cons
   P.b.split = I;
   P.offsets = offsets;
   P.G = G;
+  P.M = A;
   P.K = H;
   P.N = 2 * I;
   P.I = I;
@@ -2377,6 +2416,7 @@ int PMX_GEMM_FN(pmx_gemm_fc2_dgrad_swiglu_bwd)(const void* dY, const void* w_dow
   P.b = one(w_down, H * I, I);
   P.offsets = offsets;
   P.G = G;
+  P.M = A;
   P.N = I;
   P.K = H;
   P.I = I;

@@ -1,0 +1,98 @@
+"""The few-rows grouped GEMM (64- and 128-row tiles) against the 256-row
+kernels and fp32 products.
+
+Calls whose copies hold few rows on average go to another kernel than the
+rest; the build ``libplacemoe_amd_w8.so`` keeps the 256-row kernels for every
+call.  Both must agree within the bf16 bar over every form the rule accepts:
+copies that end on and next to the tile edges (64, 128), empty copies, one
+copy, as many as the kernel takes (1024) and one more (which goes to the other
+kernels), K off the 64-deep K-tile, columns off the 256-wide tile, split fc1
+weights whose split is (and is not) a whole number of K-tiles, and top-1 row
+maps with targets outside the output.
+"""
+
+import numpy as np
+import pytest
+import torch
+
+from placemoe_amd import _capi, build, kernels
+from tests.helpers import assert_bf16_close
+from tests.test_gpu_gemm_random_layouts import check_every_kind
+
+pytestmark = pytest.mark.gpu
+
+EDGES = [1, 0, 15, 16, 17, 63, 64, 65, 0, 2, 127, 128, 129, 31, 33, 5]
+
+
+def _off(counts):
+    off = np.zeros(len(counts) + 1, dtype=np.int64)
+    np.cumsum(counts, out=off[1:])
+    return off
+
+
+def _sparse(G, seed):
+    c = np.zeros(G, dtype=np.int64)
+    rng = np.random.default_rng(seed)
+    c[rng.choice(G, 20, replace=False)] = rng.integers(1, 150, 20)
+    c[0], c[-1] = 3, 66
+    return c
+
+
+CASES = {
+    "tiny": ([3, 0, 1, 7, 0, 9], 512, 192),
+    "edges": (EDGES, 576, 264),
+    "edges128": ([128, 127, 129, 60, 200, 100], 320, 136),
+    "k_tail": (EDGES, 200, 72),
+    "one_copy": ([37], 1024, 640),
+    "one_k_tile": ([5, 70, 0, 12], 64, 64),
+    "below_one_k_tile": ([5, 70, 0, 12], 40, 24),
+    "g1024": (_sparse(1024, 1), 128, 72),
+    "g1025": (_sparse(1025, 2), 128, 72),
+}
+
+
+@pytest.mark.parametrize("name", list(CASES))
+def test_every_kind_against_fp32(cuda, name):
+    counts, H, I = CASES[name]
+    print(f"few rows {name}: G={len(counts)} rows={int(np.sum(counts))} H={H} I={I}", flush=True)
+    check_every_kind(cuda, _off(counts), H, I, 21, name)
+
+
+def _outputs(cuda, counts, H, I, dtype):
+    off = _off(counts)
+    G, A = len(counts), int(off[-1])
+    offd = torch.as_tensor(off, dtype=torch.int32, device=cuda)
+    gen = torch.Generator(device=cuda).manual_seed(4)
+
+    def rn(*shape, scale=1.0):
+        return (torch.randn(shape, generator=gen, device=cuda) * scale).to(dtype)
+
+    x, dy = rn(A, H), rn(A, H)
+    w1, w2 = rn(G, 2 * I, H, scale=0.05), rn(G, H, I, scale=0.05)
+    perm = torch.randperm(A, generator=gen, device=cuda).to(torch.int32)
+    perm[::7] = A + 3  # targets outside the output are dropped
+    perm[3::11] = -1
+    rw = (0.05 + 0.95 * torch.rand((A,), generator=gen, device=cuda)).to(dtype)
+    gate, up = w1[:, :I].contiguous(), w1[:, I:].contiguous()
+    gu, act = kernels.gemm_fc1_swiglu(x, gate, up, I * H, offd, G, I)
+    keep = perm[(perm >= 0) & (perm < A)].long()
+    y, out = kernels.group_gemm_nt_combine_top1(act, w2, offd, perm, rw)
+    dg1 = kernels.gemm_fc2_dgrad_swiglu(dy, w2, gu, offd)
+    return {"gu": gu, "act": act, "y": y, "out": out[keep], "dg1": dg1, "dact": kernels.group_gemm_nn(dy, w2, offd),
+            "dxp": kernels.group_gemm_nn(dg1, gate, offd, b_second=up),
+            "dx": kernels.group_gemm_nn_unpermute_top1(dg1, w1, offd, perm)[keep]}
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
+@pytest.mark.parametrize("name", list(CASES))
+def test_same_as_the_256_row_kernels(cuda, name, dtype):
+    variant = build.variant_path("w8")
+    assert variant.exists(), f"{variant} is not built (python -m placemoe_amd.build)"
+    counts, H, I = CASES[name]
+    print(f"few rows against 256-row kernels, {name} {dtype}", flush=True)
+    got = _outputs(cuda, counts, H, I, dtype)
+    with _capi.using(variant):
+        ref = _outputs(cuda, counts, H, I, dtype)
+    torch.cuda.synchronize()
+    for k in ref:
+        assert_bf16_close(got[k], ref[k], name=f"{name} {k}")
