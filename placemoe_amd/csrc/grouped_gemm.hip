@@ -354,8 +354,9 @@ __device__ __forceinline__ void issue_one(char* stage, const Tile<KIND, BM>& tc,
 // RS: piece Q0 (A pieces 0 .. QA-1, then B) of this wave's share of K-tile
 // kt, loaded into a register with the addressing of the buffer->LDS
 // instruction it replaces (FAST ragged-M kinds), and its store to the LDS
-// position that instruction fills.
-template <int KIND, int BM, int PIECE>
+// position that instruction fills.  TWO (fc1 dgrad with split weights, the
+// split a whole number of K-tiles): K-tiles from the split on come from r1.
+template <int KIND, int BM, int PIECE, bool TWO>
 __device__ __forceinline__ uint4 load_piece(const Tile<KIND, BM>& tc, int32_t kt, int wave) {
   constexpr int QA = loads_per_wave<BM>();
   if constexpr (PIECE < QA) {
@@ -364,13 +365,20 @@ __device__ __forceinline__ uint4 load_piece(const Tile<KIND, BM>& tc, int32_t kt
   } else {
     constexpr int Q0 = PIECE - QA;
     uint32_t soff;
+    __amdgpu_buffer_rsrc_t r = tc.B.r0;
     if constexpr (b_is_mn<KIND>()) {
       constexpr int ROWS = 1024 / (2 * BN);
       soff = ((uint32_t)kt * BK + (uint32_t)((Q0 * NWAVES + wave) * ROWS)) * tc.B.ldb;
+      if constexpr (TWO) {
+        if (kt * BK >= tc.B.split) {
+          r = tc.B.r1;
+          soff -= tc.B.split_bytes;
+        }
+      }
     } else {
       soff = (uint32_t)kt * (BK * 2);
     }
-    return __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(tc.B.r0, tc.B.voff[Q0], soff, 0));
+    return __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(r, tc.B.voff[Q0], soff, 0));
   }
 }
 template <int BM, int PIECE>
@@ -1110,11 +1118,13 @@ __device__ __forceinline__ void group_prefix(const GemmParams& P, int32_t* tpre,
 // p+2, so every load has a whole K-tile to land and the loads are spread
 // over the K-tile instead of crowding its first half; the compiler tracks
 // these loads, and the end of a K-tile waits only for LDS.
-template <int KIND, int BM, bool BAL = false, bool FAST = false, bool RS = false>
+// TWO (RS fc1 dgrad): the weights are two tensors that meet at a K-tile.
+template <int KIND, int BM, bool BAL = false, bool FAST = false, bool RS = false, bool TWO = false>
 __global__ __launch_bounds__(NTHREADS, 1) void grouped_gemm_kernel(GemmParams P) {
   static_assert(!BAL || KIND == KIND_TN, "the balanced order is the weight gradient's");
   static_assert(!RS || (FAST && (KIND == KIND_FC1 || KIND == KIND_NT || KIND == KIND_NN)),
                 "register-staged operands: FAST ragged-M kinds without the SwiGLU backward");
+  static_assert(!TWO || (RS && KIND == KIND_NN), "two weight tensors: register-staged fc1 dgrad");
   static_assert(BM == 256, "the schedule below is written for 256 x 256 tiles");
   static_assert(BK == pmx::kKTileRows, "wgrad K-tile windows are 64 rows deep");
   constexpr int STAGE_BYTES = (BM + BN) * BK * 2;
@@ -1272,12 +1282,12 @@ __global__ __launch_bounds__(NTHREADS, 1) void grouped_gemm_kernel(GemmParams P)
   int cs = 0;  // stage of the K-tile being multiplied
   if constexpr (RS) {
     static_for<0, NPC>([&](auto q) __attribute__((always_inline)) {
-      rg[decltype(q)::value] = load_piece<KIND, BM, decltype(q)::value>(it, i_kt, wave);
+      rg[decltype(q)::value] = load_piece<KIND, BM, decltype(q)::value, TWO>(it, i_kt, wave);
     });
     advance_issue();
     static_for<0, NPC>([&](auto q) __attribute__((always_inline)) {
       store_piece<BM, decltype(q)::value>(lds, wave, lane, rg[decltype(q)::value]);
-      rg[decltype(q)::value] = load_piece<KIND, BM, decltype(q)::value>(it, i_kt, wave);
+      rg[decltype(q)::value] = load_piece<KIND, BM, decltype(q)::value, TWO>(it, i_kt, wave);
     });
     advance_issue();
     wait_lds();
@@ -1316,7 +1326,7 @@ __global__ __launch_bounds__(NTHREADS, 1) void grouped_gemm_kernel(GemmParams P)
   auto rs_piece = [&](auto pc, char* refill) __attribute__((always_inline)) {
     constexpr int q = decltype(pc)::value;
     store_piece<BM, q>(refill, wave, lane, rg[q]);
-    rg[q] = load_piece<KIND, BM, q>(it, i_kt, wave);
+    rg[q] = load_piece<KIND, BM, q, TWO>(it, i_kt, wave);
   };
   // k-step KS of the current K-tile: MFMAs of k-step KS-1 (fragments `fm`)
   // interleaved with the reads of k-step KS into `fr`, and, with LOADS, the
@@ -2271,6 +2281,17 @@ int launch(const GemmParams& P, hipStream_t stream) {
       }
     }
     if (!fast) {
+      if constexpr (KIND == KIND_NN) {
+        // Split fc1 weights that meet at a K-tile: the register-staged loads,
+        // which pick the tensor per K-tile (the general path masks and selects
+        // per load: 128 copies of 256 rows of the 2048 x 768 layer 333 -> 291 us,
+        // 160 of 819 rows 887 -> 825, 16 of 4096 rows of 7168 x 2048 3252 -> 3148).
+        if (P.K % BK == 0 && P.b.split % BK == 0) {
+          grouped_gemm_kernel<KIND, kBM, false, true, true, true><<<grid, NTHREADS, 0, stream>>>(P);
+          PMX_LAUNCH_CHECK();
+          return PMX_OK;
+        }
+      }
       grouped_gemm_kernel<KIND, kBM><<<grid, NTHREADS, 0, stream>>>(P);
     } else if constexpr (KIND == KIND_FC1 || KIND == KIND_NT) {
       grouped_gemm_kernel<KIND, kBM, false, true, true><<<grid, NTHREADS, 0, stream>>>(P);
