@@ -2201,28 +2201,33 @@ template <int KIND>
 constexpr bool use_w4() { return PMX_GEMM_W4 && ((PMX_W4_KINDS >> KIND) & 1); }
 
 // Copies with few rows (few_rows.h).  The host knows the average rows per copy,
-// M / G, not the counts.  Up to kFewRows64 rows on average 64 x 256 tiles, up
-// to kFewRows128 128 x 256 tiles, beyond that the kernels above, whose
-// 256-row tiles read each weight strip for twice the rows.  Where the lines
-// lie (us; 64-row / 128-row tiles / 256-row kernels; 128 or 160 copies of the
-// 2048 x 768 layer, row counts log-normal with sigma 0.5):
-//   rows    fc1             fc2             fc2 dgrad       fc1 dgrad
-//   4.8     177 / 178 / 267  90 /  92 / 108  90 /  92 / 140 169 / 171 / 204
-//   25      187 / 191 / 267 107 /  99 / 105 108 / 110 / 145 194 / 184 / 196
-//   96      223 / 211 / 268 119 / 116 / 109 130 / 119 / 144 199 / 196 / 196
-//   150     266 / 227 / 270 156 / 129 / 115 178 / 160 / 152 252 / 216 / 210
-//   256     366 / 300 / 328 228 / 181 / 148 240 / 207 / 221 360 / 288 / 267
-// fc1 and the fc2 dgrad run on the four-wave kernel, whose loads have one
-// K-tile to land, and gain the most; fc2 and the fc1 dgrad on the
-// register-staged kernel (two K-tiles).  PMX_FEW_ROWS=0 builds without it (the
-// test variants of the 256-row kernels).
+// M / G, not the counts; two tilings:
+//   64 x 128, two blocks per CU: fc1 and fc2 up to kFewRows64 rows, and the
+//     dgrads where 256-wide tiles would be fewer than the CUs (at most
+//     min(G, M) copies have rows);
+//   128 x 256, one block: up to kFewRows128 rows (the dgrads' [K][N] weights
+//     prefer its 512-byte row segments).
+// Beyond that the kernels above, whose 256-row tiles read each weight strip
+// for twice the rows.  Where the lines lie (us; 64 x 128 / 128 x 256 / 256-row
+// kernels; 2048 x 768 layer, row counts log-normal with sigma 0.5):
+//   copies rows  fc1             fc2             fc2 dgrad       fc1 dgrad
+//   160    4.8   183 / 189 / 265  90 /  91 / 104  95 /  94 / 147 185 / 172 / 193
+//   160    25    194 / 193 / 269 104 / 110 / 107 110 / 108 / 146 207 / 196 / 204
+//   128    96    215 / 198 / 263 119 / 119 / 120 131 / 119 / 141 219 / 198 / 204
+//   128    150   265 / 227 / 270 152 / 129 / 115 167 / 160 / 152 263 / 216 / 210
+//   128    256   382 / 300 / 328 221 / 181 / 148 246 / 207 / 221 383 / 288 / 267
+// and for 16 copies of 7168 x 2048, 12 rows: 159 / 158 / 218, 98 / 100 / 116,
+// 84 / 110 / 184 (a narrow one), 178 / 164 / 193.  fc1 and the fc2 dgrad gain
+// the most: their 256-row kernel's loads have one K-tile to land, those of
+// the register-staged one, which runs fc2 and the fc1 dgrad, two.
+// PMX_FEW_ROWS=0 builds without it (the test variants of the 256-row kernels).
 #ifndef PMX_FEW_ROWS
 #define PMX_FEW_ROWS 1
 #endif
-using Few64 = fr::Cfg<1, 8, 4, 2, 2, 3, 1>;   // 64 x 256 tiles, 40 KB stages
+using Few64 = fr::Cfg<1, 4, 4, 2, 2, 3, 2>;   // 64 x 128 tiles, 24 KB stages
 using Few128 = fr::Cfg<2, 4, 4, 4, 2, 3, 1>;  // 128 x 256 tiles, 48 KB stages
-constexpr int64_t kFewRows64[4] = {40, 16, 16, 40};     // fc1, fc2, fc1 dgrad, fc2 dgrad
-constexpr int64_t kFewRows128[4] = {224, 48, 64, 120};
+constexpr int64_t kFewRows64[4] = {40, 48, 40, 40};  // fc1, fc2, fc1 dgrad, fc2 dgrad
+constexpr int64_t kFewRows128[4] = {224, 48, 40, 120};
 
 template <int KIND, class CF>
 int launch_few(const GemmParams& P, int cus, hipStream_t stream) {
@@ -2265,7 +2270,9 @@ int launch(const GemmParams& P, hipStream_t stream) {
   } else {
     // Weights in two tensors: the few-rows kernel picks one per K-tile.
     const bool few = PMX_FEW_ROWS && P.G <= fr::kMaxG && (KIND != KIND_NN || P.b.split >= P.K || P.b.split % BK == 0);
-    if (few && P.M <= kFewRows64[KIND] * P.G) return launch_few<KIND, Few64>(P, grid, stream);
+    const int64_t copies = P.M < P.G ? P.M : P.G;
+    const bool narrow = KIND == KIND_FC1 || KIND == KIND_NT || copies * ((P.N + BN - 1) / BN) < grid;
+    if (few && narrow && P.M <= kFewRows64[KIND] * P.G) return launch_few<KIND, Few64>(P, grid, stream);
     if (few && P.M <= kFewRows128[KIND] * P.G) return launch_few<KIND, Few128>(P, grid, stream);
     // FAST: K a multiple of 64, dgrad weights not split (P.b.split >= K).
     // RS (register-staged operands): fc1 and fc2 always; the fc1 dgrad when

@@ -42,6 +42,9 @@ CASES = {
     "tiny": ([3, 0, 1, 7, 0, 9], 512, 192),
     "edges": (EDGES, 576, 264),
     "edges128": ([128, 127, 129, 60, 200, 100], 320, 136),
+    "edges128_tile": ([128, 127, 129, 60, 200, 100], 320, 192),
+    "edges32": ([129, 1, 0, 64, 2, 3, 17, 40], 576, 192),
+    "wide": ([1 + i % 29 for i in range(80)] + [0, 63, 64, 65, 128], 1096, 776),
     "k_tail": (EDGES, 200, 72),
     "one_copy": ([37], 1024, 640),
     "one_k_tile": ([5, 70, 0, 12], 64, 64),
