@@ -209,6 +209,18 @@ __global__ __launch_bounds__(1024) void route_scan_kernel(int32_t* __restrict__ 
   if (tid == 0) status[0] = bad_sh;
 }
 
+// Assignments of a wave equal to each lane's (bits over the lanes; an invalid
+// lane equals nothing).
+__device__ __forceinline__ uint64_t match_any(int32_t v, bool valid, int nbits) {
+  uint64_t mask = __ballot(valid);
+  for (int b = 0; b < nbits; ++b) {
+    const bool bit = (v >> b) & 1;
+    const uint64_t m = __ballot(bit);
+    mask &= bit ? m : ~m;
+  }
+  return mask;
+}
+
 // One wave per chunk: stable rank of every assignment among equal copies.
 template <bool USE_LDS>
 __global__ __launch_bounds__(64) void route_rank_kernel(const int32_t* __restrict__ phys,
@@ -231,12 +243,7 @@ __global__ __launch_bounds__(64) void route_rank_kernel(const int32_t* __restric
     const int64_t a = seg + lane;
     const bool valid = a < end;
     const int32_t v = valid ? phys[a] : 0;
-    uint64_t mask = __ballot(valid);
-    for (int b = 0; b < nbits; ++b) {
-      const bool bit = (v >> b) & 1;
-      const uint64_t m = __ballot(bit);
-      mask &= bit ? m : ~m;
-    }
+    const uint64_t mask = match_any(v, valid, nbits);
     int32_t base = 0;
     if (valid) {
       // The global-table counters are read and written by this wave only;
@@ -253,6 +260,117 @@ __global__ __launch_bounds__(64) void route_rank_kernel(const int32_t* __restric
       }
     }
     __syncthreads();
+  }
+}
+
+// The whole routing path of a small batch in one block: 16 waves, each a chunk
+// of `chunk` assignments (a multiple of 64) with its histogram row in LDS; the
+// columns are scanned over the waves and the copies in LDS, and each wave then
+// ranks its chunk.  The three-kernel path costs three launches whatever the
+// size; one block's walk grows with A (us in a replayed graph, one block /
+// three kernels; 128-160 copies unless stated): 8 assignments 5.1 / 8.0, 768
+// 5.8 / 14.8, 4096 7.7 / 16.6, 8192 over 12 copies 10.4 / 14.4, 12248 16.2 /
+// 16.8, 32768 37.6 / 16.5.
+constexpr int kSmallWaves = 16;
+constexpr int64_t kSmallMaxAssign = 8192;
+constexpr int kSmallMaxSlots = 896;  // (16 + 1) x C counters in 64 KB of LDS
+
+__global__ __launch_bounds__(64 * kSmallWaves) void route_small_kernel(
+    const int64_t* __restrict__ sel, const int64_t* __restrict__ M, const int64_t* __restrict__ src,
+    int32_t src_const, int32_t S, int32_t E, int32_t K, int32_t C, int32_t A, int32_t chunk, int nbits,
+    int32_t* __restrict__ phys, int32_t* __restrict__ counts, int32_t* __restrict__ offsets,
+    int32_t* __restrict__ pos, int32_t* __restrict__ status) {
+  extern __shared__ int32_t hist[];  // [16][C]: the waves' histograms, then their next positions
+  __shared__ int32_t wave_sums[kSmallWaves];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  for (int i = tid; i < kSmallWaves * C; i += 64 * kSmallWaves) hist[i] = 0;
+  __syncthreads();
+  int32_t* row = hist + wave * C;
+  const int32_t begin = wave * chunk < A ? wave * chunk : A;
+  const int32_t end = begin + chunk < A ? begin + chunk : A;
+  int bad = 0;
+  constexpr int U = 4;  // segments of 64 loaded together
+  for (int32_t a0 = begin + lane; a0 < end; a0 += 64 * U) {
+    int64_t e[U], s[U], c[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int32_t a = a0 + 64 * u;
+      e[u] = a < end ? sel[a] : 0;
+      s[u] = (int64_t)src_const;
+      if (src != nullptr && a < end) s[u] = src[a / K];
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const bool in = a0 + 64 * u < end;
+      c[u] = e[u];
+      if (M != nullptr) {
+        if (s[u] < 0 || s[u] >= S) { bad |= in; s[u] = s[u] < 0 ? 0 : S - 1; }
+        if (e[u] < 0 || e[u] >= E) { bad |= in; e[u] = e[u] < 0 ? 0 : E - 1; }
+        c[u] = M[s[u] * E + e[u]];
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int32_t a = a0 + 64 * u;
+      if (a < end) {
+        if (c[u] < 0 || c[u] >= C) { bad = 1; c[u] = c[u] < 0 ? 0 : C - 1; }
+        phys[a] = (int32_t)c[u];
+        atomicAdd(&row[c[u]], 1);
+      }
+    }
+  }
+  const int any_bad = __syncthreads_or(bad);
+  // Thread c: copy c's total over the waves, then the exclusive scan over the copies.
+  int32_t total = 0;
+  if (tid < C)
+    for (int w = 0; w < kSmallWaves; ++w) total += hist[w * C + tid];
+  int32_t inc = total;
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) {
+    const int32_t v = __shfl_up(inc, off, 64);
+    if (lane >= off) inc += v;
+  }
+  if (lane == 63) wave_sums[wave] = inc;
+  __syncthreads();
+  int32_t start = inc - total;
+  for (int w = 0; w < wave; ++w) start += wave_sums[w];
+  if (tid < C) {
+    counts[tid] = total;
+    offsets[tid] = start;
+    int32_t run = start;
+    for (int w = 0; w < kSmallWaves; ++w) {
+      const int32_t v = hist[w * C + tid];
+      hist[w * C + tid] = run;
+      run += v;
+    }
+  }
+  if (tid == 0) {
+    offsets[C] = A;
+    status[0] = any_bad ? 1 : 0;
+  }
+  __syncthreads();
+  // Stable ranks.  Only this wave touches its row from here on, and a wave's
+  // LDS accesses take effect in order; the waits keep the compiler from
+  // moving them past each other.
+  const uint64_t lt_mask = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
+  for (int32_t a0 = begin + lane; a0 - lane < end; a0 += 64 * U) {
+    int32_t v[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) v[u] = a0 + 64 * u < end ? phys[a0 + 64 * u] : 0;  // this lane's own stores
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int32_t a = a0 + 64 * u;
+      const bool valid = a < end;
+      const uint64_t mask = match_any(v[u], valid, nbits);
+      const int32_t base = valid ? __hip_atomic_load(&row[v[u]], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) : 0;
+      __builtin_amdgcn_wave_barrier();
+      if (valid) {
+        pos[a] = base + __popcll(mask & lt_mask);
+        if (lane == 63 - __clzll(mask))
+          __hip_atomic_store(&row[v[u]], base + __popcll(mask), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+      }
+      __builtin_amdgcn_wave_barrier();
+    }
   }
 }
 
@@ -278,6 +396,15 @@ int launch_route(const int64_t* sel, const int64_t* M, const int64_t* src, int32
   int32_t* flags = table + g.nchunks * (int64_t)C;
   const bool lds = C <= kRouteLdsMaxSlots;
   const size_t lds_bytes = lds ? (size_t)C * sizeof(int32_t) : 0;
+  int nbits = 1;
+  while ((1 << nbits) < C) ++nbits;
+  if (A > 0 && A <= kSmallMaxAssign && C <= kSmallMaxSlots) {
+    const int32_t chunk = (int32_t)((A + 64 * kSmallWaves - 1) / (64 * kSmallWaves)) * 64;
+    route_small_kernel<<<1, 64 * kSmallWaves, (size_t)kSmallWaves * C * sizeof(int32_t), stream>>>(
+        sel, M, src, src_const, S, E, K, C, (int32_t)A, chunk, nbits, phys, counts, offsets, pos, status);
+    PMX_LAUNCH_CHECK();
+    return PMX_OK;
+  }
   if (A == 0) {
     // No assignments: the table is one zero row and its chunk flag (which
     // follows it) is clear; the scan still writes counts, offsets and the
@@ -294,8 +421,6 @@ int launch_route(const int64_t* sel, const int64_t* M, const int64_t* src, int32
   route_scan_kernel<<<1, 1024, 0, stream>>>(table, g.nchunks, C, flags, counts, offsets, status);
   PMX_LAUNCH_CHECK();
   if (A > 0) {
-    int nbits = 1;
-    while ((1 << nbits) < C) ++nbits;
     if (lds) {
       route_rank_kernel<true><<<(unsigned)g.nchunks, 64, lds_bytes, stream>>>(phys, table, C, A, g.chunk,
                                                                              nbits, pos);
@@ -396,6 +521,34 @@ __global__ __launch_bounds__(kRowThreads) void gather_rows_by_src_kernel(const b
   const uint4* src = reinterpret_cast<const uint4*>(X + (ok ? t : 0) * H);
   uint4* dst = reinterpret_cast<uint4*>(Xp + r * H);
   for (int64_t i = threadIdx.x; i < n8; i += blockDim.x) st_stream(dst + i, ok ? ld_stream(src + i) : make_uint4(0, 0, 0, 0));
+}
+
+// The same for few rows in one launch instead of three (the map's fill, the
+// inversion, the copy: 4-5 us each whatever the size): block r finds its
+// token by searching pos, T x 4 bytes from L2.
+constexpr int64_t kFindMaxRows = 1024;
+__global__ __launch_bounds__(kRowThreads) void permute_top1_few_kernel(const bf16_t* __restrict__ X,
+                                                                       const int32_t* __restrict__ pos,
+                                                                       const bf16_t* __restrict__ w, int32_t T,
+                                                                       int64_t H, bf16_t* __restrict__ Xp,
+                                                                       int32_t* __restrict__ row_src,
+                                                                       bf16_t* __restrict__ row_w) {
+  __shared__ int32_t found;
+  const int32_t r = blockIdx.x;
+  if (threadIdx.x == 0) found = -1;
+  __syncthreads();
+  for (int32_t t = threadIdx.x; t < T; t += blockDim.x)
+    if (pos[t] == r) atomicMax(&found, t);
+  __syncthreads();
+  const int32_t t = found;
+  if (threadIdx.x == 0) {
+    row_src[r] = t;
+    if (row_w != nullptr && t >= 0) row_w[r] = w[t];
+  }
+  const int64_t n8 = H / 8;
+  const uint4* src = reinterpret_cast<const uint4*>(X + (int64_t)(t >= 0 ? t : 0) * H);
+  uint4* dst = reinterpret_cast<uint4*>(Xp + r * H);
+  for (int64_t i = threadIdx.x; i < n8; i += blockDim.x) st_stream(dst + i, t >= 0 ? ld_stream(src + i) : make_uint4(0, 0, 0, 0));
 }
 
 // out[t] = bf16( sum_k fp32(term_k) ), term_k = Y[pos] or bf16(Y[pos] * w).
@@ -822,7 +975,10 @@ int pmx_moe_scatter_src(const void* X, const int32_t* pos, const void* w, int64_
   const bf16_t* wb = static_cast<const bf16_t*>(w);
   bf16_t* rw = static_cast<bf16_t*>(row_w);
   if (H % 8 == 0 && aligned16(X) && aligned16(Xp)) {
-    if (K == 1 && row_src != nullptr) {
+    if (K == 1 && row_src != nullptr && T <= kFindMaxRows) {
+      permute_top1_few_kernel<<<(unsigned)T, th, 0, stream>>>((const bf16_t*)X, pos, wb, (int32_t)T, H, (bf16_t*)Xp,
+                                                              row_src, rw);
+    } else if (K == 1 && row_src != nullptr) {
       // top-1 with the row map: the map first (every row -1, then the rows
       // pos names), then the rows in storage order
       fill_i32_kernel<<<(unsigned)((T + 255) / 256), 256, 0, stream>>>(row_src, T, -1);
