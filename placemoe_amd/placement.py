@@ -286,11 +286,11 @@ class LayerPlacement:
     def record_slot_tokens(self, counts: torch.Tensor) -> None:
         """Accumulate per-copy token counts on the device (no host sync);
         ``record_local_expert_token_counts``, expert_swap.py:6200-6218."""
-        counts = counts.detach().to(torch.int64)
+        counts = counts.detach()
         if self.accumulated_slot_tokens is None or self.accumulated_slot_tokens.shape != counts.shape:
-            self.accumulated_slot_tokens = counts.clone()
+            self.accumulated_slot_tokens = counts.to(torch.int64, copy=True)
         else:
-            self.accumulated_slot_tokens.add_(counts)
+            self.accumulated_slot_tokens.add_(counts)  # int32 counts into the int64 sums: one kernel
 
     def clear_slot_tokens(self) -> None:
         self.accumulated_slot_tokens = None
