@@ -68,8 +68,8 @@ EXTRA_OBJECTS = {"grouped_gemm.f16": ("grouped_gemm.hip", ["-DPMX_ELT_F16"])}
 # name -> (source, extra flags): library variants for tests and comparisons.
 #   tiletab2: a two-entry LDS tile table (the on-the-spot tile decode runs at small shapes);
 #   w8:       the eight-wave GEMM kernel for every call (the four-wave kernel switched off).
-# Both build without the few-rows kernel, so that small shapes reach the 256-row kernels they are for.
-VARIANTS = {"tiletab2": ("grouped_gemm.hip", ["-DPMX_TILE_TAB=2", "-DPMX_FEW_ROWS=0"]),
+#             It builds without the few-rows kernel too, so that small shapes reach the 256-row kernels.
+VARIANTS = {"tiletab2": ("grouped_gemm.hip", ["-DPMX_TILE_TAB=2"]),
             "w8": ("grouped_gemm.hip", ["-DPMX_GEMM_W4=0", "-DPMX_FEW_ROWS=0"])}
 VARIANT_DIR = LIB_DIR / "variants"
 

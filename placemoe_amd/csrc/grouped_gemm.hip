@@ -2211,23 +2211,23 @@ constexpr bool use_w4() { return PMX_GEMM_W4 && ((PMX_W4_KINDS >> KIND) & 1); }
 // for twice the rows.  Where the lines lie (us; 64 x 128 / 128 x 256 / 256-row
 // kernels; 2048 x 768 layer, row counts log-normal with sigma 0.5):
 //   copies rows  fc1             fc2             fc2 dgrad       fc1 dgrad
-//   160    4.8   183 / 189 / 265  90 /  91 / 104  95 /  94 / 147 185 / 172 / 193
-//   160    25    194 / 193 / 269 104 / 110 / 107 110 / 108 / 146 207 / 196 / 204
-//   128    96    215 / 198 / 263 119 / 119 / 120 131 / 119 / 141 219 / 198 / 204
-//   128    150   265 / 227 / 270 152 / 129 / 115 167 / 160 / 152 263 / 216 / 210
-//   128    256   382 / 300 / 328 221 / 181 / 148 246 / 207 / 221 383 / 288 / 267
-// and for 16 copies of 7168 x 2048, 12 rows: 159 / 158 / 218, 98 / 100 / 116,
+//   160    4.8   180 / 175 / 265  90 /  91 / 104  95 /  94 / 147 185 / 172 / 193
+//   160    25    185 / 185 / 269 103 / 108 / 107 110 / 108 / 146 207 / 196 / 204
+//   128    96    213 / 195 / 263 119 / 118 / 120 131 / 119 / 141 219 / 198 / 204
+//   128    150   263 / 222 / 270 152 / 129 / 115 167 / 160 / 152 263 / 216 / 210
+//   128    256   391 / 304 / 328 221 / 179 / 148 246 / 207 / 221 383 / 288 / 267
+// and for 16 copies of 7168 x 2048, 12 rows: 159 / 159 / 218, 86 / 83 / 116,
 // 84 / 110 / 184 (a narrow one), 178 / 164 / 193.  fc1 and the fc2 dgrad gain
 // the most: their 256-row kernel's loads have one K-tile to land, those of
 // the register-staged one, which runs fc2 and the fc1 dgrad, two.
-// PMX_FEW_ROWS=0 builds without it (the test variants of the 256-row kernels).
+// PMX_FEW_ROWS=0 builds without it (the eight-wave test variant).
 #ifndef PMX_FEW_ROWS
 #define PMX_FEW_ROWS 1
 #endif
 using Few64 = fr::Cfg<1, 4, 4, 2, 2, 3, 2>;   // 64 x 128 tiles, 24 KB stages
 using Few128 = fr::Cfg<2, 4, 4, 4, 2, 3, 1>;  // 128 x 256 tiles, 48 KB stages
 constexpr int64_t kFewRows64[4] = {40, 48, 40, 40};  // fc1, fc2, fc1 dgrad, fc2 dgrad
-constexpr int64_t kFewRows128[4] = {224, 48, 40, 120};
+constexpr int64_t kFewRows128[4] = {208, 48, 40, 120};
 
 template <int KIND, class CF>
 int launch_few(const GemmParams& P, int cus, hipStream_t stream) {
@@ -2280,8 +2280,15 @@ int launch(const GemmParams& P, hipStream_t stream) {
     // weight strip serves few tiles and its loads wait on memory - with a
     // few large copies the DMA path is faster (it spends less power).
     const bool fast = P.K % BK == 0 && (KIND != KIND_NN || P.b.split >= P.K);
+    // fc1 with up to kRsFc1Rows rows per copy: the register-staged loads, with
+    // two K-tiles to land, as for fc2 and the fc1 dgrad (us, register-staged /
+    // four-wave: 128 copies of 256 rows of 2048 x 768 302 / 325, 400 rows 404 /
+    // 414-444, 32 copies of 500 rows of 4096 x 1536 421-430 / 428-437; past it
+    // the four-wave kernel: 160 copies of 819 rows 856-870 / 824-861).
+    constexpr int64_t kRsFc1Rows = 600;
+    [[maybe_unused]] const bool rs_fc1 = KIND == KIND_FC1 && P.M <= kRsFc1Rows * P.G;
     if constexpr (use_w4<KIND>()) {
-      if (fast) {
+      if (fast && !rs_fc1) {
         w4::grouped_gemm_w4_kernel<KIND><<<grid, w4::NT, 0, stream>>>(P);
         PMX_LAUNCH_CHECK();
         return PMX_OK;
