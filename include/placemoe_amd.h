@@ -185,6 +185,17 @@ int pmx_gemm_fc1_swiglu_fwd(const void* X, const void* w_gate, const void* w_up,
                             int64_t A, int64_t H, int64_t I, void* gu, void* act,
                             pmx_stream_t stream);
 
+/* pmx_gemm_fc1_swiglu_fwd that writes each row's activation times its router
+ * weight, act_w[a] = bf16( act[a] * row_w[a] ), in act's place: the fc2 input
+ * of the reference's non-EP arithmetic, equal to pmx_gemm_fc1_swiglu_fwd
+ * followed by pmx_weight_rows bit for bit.  row_w bf16 [A] (see
+ * pmx_moe_scatter_src).  Replaces group_gemm.py:236-276 (split), :480-499
+ * (merged). */
+int pmx_gemm_fc1_swiglu_weighted_fwd(const void* X, const void* w_gate, const void* w_up,
+                                     int64_t w_copy_stride, const int32_t* offsets, int32_t G,
+                                     int64_t A, int64_t H, int64_t I, const void* row_w, void* gu,
+                                     void* act_w, pmx_stream_t stream);
+
 /* Ragged-M grouped GEMM, B transposed: C[a] = bf16(A[a] @ B[g]^T), B [G,N,K].
  * Forward fc2 (A = act, B = down_proj [G,H,I]).
  * Replaces group_gemm_same_nk(transpose_b=True)
@@ -283,6 +294,12 @@ int pmx_weight_rows(const void* act, const void* row_w, int64_t R, int64_t N, vo
 int pmx_swiglu_bwd_weighted(const void* d_act_w, const void* gu, const void* act, const void* row_w,
                             const int32_t* row_src, int64_t R, int64_t I, int64_t A, void* dG1,
                             void* dw, pmx_stream_t stream);
+
+/* pmx_swiglu_bwd_weighted without the saved activations: act is recomputed
+ * from gu with the forward's rounding points, bit for bit what
+ * pmx_gemm_fc1_swiglu_fwd wrote for these gu. */
+int pmx_swiglu_bwd_weighted_gu(const void* d_act_w, const void* gu, const void* row_w, const int32_t* row_src,
+                               int64_t R, int64_t I, int64_t A, void* dG1, void* dw, pmx_stream_t stream);
 
 /* ------------------------------------------------------------------------ */
 /* Replica-gradient fold                                                     */
@@ -442,6 +459,10 @@ int pmx_segment_sum_f16(const void* source, const int64_t* index, int64_t N, int
 int pmx_gemm_fc1_swiglu_fwd_f16(const void* X, const void* w_gate, const void* w_up, int64_t w_copy_stride,
                                 const int32_t* offsets, int32_t G, int64_t A, int64_t H, int64_t I, void* gu,
                                 void* act, pmx_stream_t stream);
+int pmx_gemm_fc1_swiglu_weighted_fwd_f16(const void* X, const void* w_gate, const void* w_up,
+                                         int64_t w_copy_stride, const int32_t* offsets, int32_t G, int64_t A,
+                                         int64_t H, int64_t I, const void* row_w, void* gu, void* act_w,
+                                         pmx_stream_t stream);
 int pmx_group_gemm_nt_f16(const void* A, const void* B, const int32_t* offsets, int32_t G, int64_t M,
                           int64_t N, int64_t K, void* C, pmx_stream_t stream);
 int pmx_group_gemm_nt_combine_top1_f16(const void* A, const void* B, const int32_t* offsets, int32_t G,
@@ -465,6 +486,9 @@ int pmx_weight_rows_f16(const void* act, const void* row_w, int64_t R, int64_t N
 int pmx_swiglu_bwd_weighted_f16(const void* d_act_w, const void* gu, const void* act, const void* row_w,
                                 const int32_t* row_src, int64_t R, int64_t I, int64_t A, void* dG1, void* dw,
                                 pmx_stream_t stream);
+int pmx_swiglu_bwd_weighted_gu_f16(const void* d_act_w, const void* gu, const void* row_w,
+                                   const int32_t* row_src, int64_t R, int64_t I, int64_t A, void* dG1, void* dw,
+                                   pmx_stream_t stream);
 int pmx_replica_fold_f16(void* grads, const int32_t* copy_offsets, const int32_t* copy_slots,
                          const int64_t* slot_tokens, int32_t E, int32_t C, int64_t P, float* out,
                          int32_t writeback, int32_t* status, pmx_stream_t stream);

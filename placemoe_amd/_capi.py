@@ -61,6 +61,15 @@ SIGNATURES = {
         c_int,
         [c_void_p, c_void_p, c_int64, c_int64, c_int64, c_void_p, c_void_p, c_size_t, c_void_p],
     ),
+    "pmx_gemm_fc1_swiglu_weighted_fwd": (
+        c_int,
+        [c_void_p, c_void_p, c_void_p, c_int64, c_void_p, c_int32, c_int64, c_int64, c_int64, c_void_p, c_void_p,
+         c_void_p, c_void_p],
+    ),
+    "pmx_swiglu_bwd_weighted_gu": (
+        c_int,
+        [c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_int64, c_int64, c_void_p, c_void_p, c_void_p],
+    ),
     "pmx_gemm_fc1_swiglu_fwd": (
         c_int,
         [c_void_p, c_void_p, c_void_p, c_int64, c_void_p, c_int32, c_int64, c_int64, c_int64,
@@ -140,7 +149,7 @@ F16_TWINS = (
     "pmx_moe_gather", "pmx_combine_fwd", "pmx_combine_bwd", "pmx_combine_bwd_top1_rows", "pmx_segment_sum",
     "pmx_gemm_fc1_swiglu_fwd", "pmx_group_gemm_nt", "pmx_group_gemm_nt_combine_top1", "pmx_group_gemm_nn",
     "pmx_group_gemm_nn_unpermute_top1", "pmx_gemm_fc2_dgrad_swiglu_bwd", "pmx_group_gemm_tn", "pmx_weight_rows",
-    "pmx_swiglu_bwd_weighted", "pmx_replica_fold", "pmx_ep_combine_aggregate",
+    "pmx_swiglu_bwd_weighted", "pmx_gemm_fc1_swiglu_weighted_fwd", "pmx_swiglu_bwd_weighted_gu", "pmx_replica_fold", "pmx_ep_combine_aggregate",
 )
 SIGNATURES.update({name + "_f16": SIGNATURES[name] for name in F16_TWINS})
 

@@ -172,6 +172,7 @@ __device__ __forceinline__ void epilogue(const GemmParams& P, const TileInfo& ti
     if (r >= ti.row_end) continue;
     if constexpr (KIND == KIND_FC1) {
       const int64_t I = P.I;
+      const float wt = P.row_w != nullptr ? Elt::to_f32(P.row_w[r]) : 0.f;
 #pragma unroll
       for (int nt = 0; nt < CF::FN; nt += 2) {
         const int64_t j = (int64_t)ti.ntile * (CF::BN / 2) + (wn * CF::FN + nt) * 8 + c4;
@@ -188,7 +189,16 @@ __device__ __forceinline__ void epilogue(const GemmParams& P, const TileInfo& ti
           g[e] = silu_f32(g[e]), g[e + 1] = silu_f32(g[e + 1]);
           Elt::round2(g[e], g[e + 1]);
         }
-        st4(P.act + r * I + j, pack4(g[0] * u[0], g[1] * u[1], g[2] * u[2], g[3] * u[3]));
+#pragma unroll
+        for (int e = 0; e < 4; ++e) g[e] *= u[e];
+        if (P.row_w != nullptr) {  // the weight on the rounded activation (non-EP fc2 input)
+#pragma unroll
+          for (int e = 0; e < 4; e += 2) {
+            Elt::round2(g[e], g[e + 1]);
+            g[e] *= wt, g[e + 1] *= wt;
+          }
+        }
+        st4(P.act + r * I + j, pack4(g[0], g[1], g[2], g[3]));
       }
     } else if constexpr (KIND == KIND_NNS) {
       const int64_t I = P.I;

@@ -139,6 +139,7 @@ struct GemmParams {
   // Top-1 row map (KIND_NN, KIND_NT; null: none).  KIND_NN writes output row
   // r to row row_tok[r] of c0 instead of row r.  KIND_NT writes row r to c0
   // and also cout[row_tok[r]] = bf16(0 + bf16(row * row_w[r])).
+  // KIND_FC1 with row_w: act[r] = bf16(act * row_w[r]) (row_tok null).
   const int32_t* row_tok;
   const bf16_t* row_w;
   bf16_t* cout;
@@ -565,6 +566,27 @@ __device__ __forceinline__ uint4 win_load(const OutWin& w, uint32_t voff, uint32
   return __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(w.r, voff + row * w.rowb, 0, kCpolNT));
 }
 
+// Eight values of a row times the row's weight, rounded: the fc2 input of the
+// non-EP arithmetic from the staged (already rounded) activations.
+__device__ __forceinline__ uint4 weighted8(const uint4& v, float w) {
+  float f[8];
+  unpack8e<Elt>(v, f);
+#pragma unroll
+  for (int j = 0; j < 8; ++j) f[j] *= w;
+  return pack8e<Elt>(f);
+}
+
+// Router weights of N rows r0 + first, + first + step, ..: the group's rows
+// from r0 on through a descriptor that ends with the group (0 past it).
+template <int N>
+__device__ __forceinline__ void row_weights(const GemmParams& P, int64_t r0, int64_t row_end, int first, int step,
+                                            float (&w)[N]) {
+  const int64_t rows = row_end - r0 < 0 ? 0 : (row_end - r0 > 256 ? 256 : row_end - r0);
+  const __amdgpu_buffer_rsrc_t rw = make_rsrc(P.row_w + r0, (uint64_t)rows * 2);
+#pragma unroll
+  for (int q = 0; q < N; ++q) w[q] = Elt::to_f32(__builtin_amdgcn_raw_buffer_load_b16(rw, (uint32_t)(first + q * step) * 2u, 0, 0));
+}
+
 template <int KIND, int BM>
 __device__ __forceinline__ void epilogue(const GemmParams& P, const TileInfo& ti, int wm, int wn, int wave, int lane,
                                          const f32x16_t (&acc)[MT][NTT], char* stage) {
@@ -604,6 +626,8 @@ __device__ __forceinline__ void epilogue(const GemmParams& P, const TileInfo& ti
       // first both as bf16 GEMM outputs (gu), then act = bf16(bf16(silu(gate)) * up).
       const int64_t I = P.I;
       const int64_t j0 = (int64_t)ti.ntile * 128 + wn * 32;
+      float rw[4];  // the act stores' rows, loaded before the first store
+      if (P.row_w != nullptr) row_weights(P, ti.row0 + rb, ti.row_end, lane >> 2, 16, rw);
       stage_half<2>(stage, wave, lane, half, [&](int mt, int nt, int i) { return acc4(acc[mt][nt], i); });
       const int cc = lane & 7;
       {
@@ -632,7 +656,11 @@ __device__ __forceinline__ void epilogue(const GemmParams& P, const TileInfo& ti
         const int64_t j = j0 + c4 * 8;
         const uint32_t voff = j < I ? (uint32_t)(lane >> 2) * w.rowb + (uint32_t)j * 2u : kOOB;
 #pragma unroll
-        for (int q = 0; q < 4; ++q) win_store(w, voff, q * 16, staged_chunk(stage, wave, q * 16 + (lane >> 2), c4));
+        for (int q = 0; q < 4; ++q) {
+          uint4 v = staged_chunk(stage, wave, q * 16 + (lane >> 2), c4);
+          if (P.row_w != nullptr) v = weighted8(v, rw[q]);
+          win_store(w, voff, q * 16, v);
+        }
       }
     } else if constexpr (KIND == KIND_NNS) {
       // fc2 dgrad: the tile is dact (bf16, as the reference stores it) for
@@ -2285,8 +2313,11 @@ int launch(const GemmParams& P, hipStream_t stream) {
     // four-wave: 128 copies of 256 rows of 2048 x 768 302 / 325, 400 rows 404 /
     // 414-444, 32 copies of 500 rows of 4096 x 1536 421-430 / 428-437; past it
     // the four-wave kernel: 160 copies of 819 rows 856-870 / 824-861).
+    // Row weights (non-EP) too: the four-wave epilogue has no register left for
+    // them (2 spill), and a separate pass over act costs more than the 1-3%
+    // between the kernels.
     constexpr int64_t kRsFc1Rows = 600;
-    [[maybe_unused]] const bool rs_fc1 = KIND == KIND_FC1 && P.M <= kRsFc1Rows * P.G;
+    [[maybe_unused]] const bool rs_fc1 = KIND == KIND_FC1 && (P.row_w != nullptr || P.M <= kRsFc1Rows * P.G);
     if constexpr (use_w4<KIND>()) {
       if (fast && !rs_fc1) {
         w4::grouped_gemm_w4_kernel<KIND><<<grid, w4::NT, 0, stream>>>(P);
@@ -2334,14 +2365,10 @@ RowSrc one(const void* p, int64_t gs, int64_t ld) {
   return s;
 }
 
-
-}  // namespace
-
-extern "C" {
-
-int PMX_GEMM_FN(pmx_gemm_fc1_swiglu_fwd)(const void* X, const void* w_gate, const void* w_up, int64_t w_copy_stride,
-                            const int32_t* offsets, int32_t G, int64_t A, int64_t H, int64_t I, void* gu,
-                            void* act, pmx_stream_t stream) {
+// fc1 + SwiGLU; row_w (or null): each row's act times its router weight.
+int fc1_swiglu(const void* X, const void* w_gate, const void* w_up, int64_t w_copy_stride, const int32_t* offsets,
+               int32_t G, int64_t A, int64_t H, int64_t I, const void* row_w, void* gu, void* act,
+               pmx_stream_t stream) {
   if (G <= 0 || G > kMaxGroups || A < 0 || H <= 0 || I <= 0) return PMX_ERR_ARG;
   if (H % 8 || I % 8 || A > INT32_MAX) return PMX_ERR_SHAPE;  // row offsets are int32
   if (A == 0) return PMX_OK;
@@ -2363,7 +2390,25 @@ int PMX_GEMM_FN(pmx_gemm_fc1_swiglu_fwd)(const void* X, const void* w_gate, cons
   P.I = I;
   P.gu = static_cast<bf16_t*>(gu);
   P.act = static_cast<bf16_t*>(act);
+  P.row_w = static_cast<const bf16_t*>(row_w);
   return launch<KIND_FC1>(P, stream);
+}
+
+}  // namespace
+
+extern "C" {
+
+int PMX_GEMM_FN(pmx_gemm_fc1_swiglu_fwd)(const void* X, const void* w_gate, const void* w_up, int64_t w_copy_stride,
+                            const int32_t* offsets, int32_t G, int64_t A, int64_t H, int64_t I, void* gu,
+                            void* act, pmx_stream_t stream) {
+  return fc1_swiglu(X, w_gate, w_up, w_copy_stride, offsets, G, A, H, I, nullptr, gu, act, stream);
+}
+
+int PMX_GEMM_FN(pmx_gemm_fc1_swiglu_weighted_fwd)(const void* X, const void* w_gate, const void* w_up,
+                                     int64_t w_copy_stride, const int32_t* offsets, int32_t G, int64_t A, int64_t H,
+                                     int64_t I, const void* row_w, void* gu, void* act_w, pmx_stream_t stream) {
+  if (A > 0 && !row_w) return PMX_ERR_ARG;
+  return fc1_swiglu(X, w_gate, w_up, w_copy_stride, offsets, G, A, H, I, row_w, gu, act_w, stream);
 }
 
 int PMX_GEMM_FN(pmx_group_gemm_nt)(const void* A, const void* B, const int32_t* offsets, int32_t G, int64_t M, int64_t N,

@@ -52,12 +52,13 @@ __device__ __forceinline__ void swiglu_bwd1(float dact, float g, float u, float&
   dup = E::round(gs) * dact;
 }
 
-// One wave per row, four rows per block.  Row r reads d_act_w[r], act[r] and
-// gu[r] (gate | up), writes dG1[r] (d_gate | d_up) and the router-weight
+// One wave per row, four rows per block.  Row r reads d_act_w[r], act[r] (null:
+// recomputed from gu with the forward's rounding points, a sixth less to read)
+// and gu[r] (gate | up), writes dG1[r] (d_gate | d_up) and the router-weight
 // gradient dw[row_src[r]] (not written when row_src[r] lies outside [0, A)).
 // The row sum: each lane sums its chunks in order (8 products per chunk, in
 // column order), then the wave's lanes are summed by a butterfly.
-template <class E, bool VEC>
+template <class E, bool VEC, bool ACT>
 __global__ __launch_bounds__(256) void swiglu_bwd_weighted_kernel(
     const bf16_t* __restrict__ daw, const bf16_t* __restrict__ gu, const bf16_t* __restrict__ act,
     const bf16_t* __restrict__ row_w, const int32_t* __restrict__ row_src, int64_t R, int64_t I, int64_t A,
@@ -76,9 +77,18 @@ __global__ __launch_bounds__(256) void swiglu_bwd_weighted_kernel(
     for (int64_t i = lane; i < n8; i += 64) {
       float d[8], a[8], g[8], u[8], dact[8], dgate[8], dup[8];
       unpack8e<E>(ld_stream(reinterpret_cast<const uint4*>(d_row) + i), d);
-      unpack8e<E>(ld_stream(reinterpret_cast<const uint4*>(a_row) + i), a);
+      if constexpr (ACT) unpack8e<E>(ld_stream(reinterpret_cast<const uint4*>(a_row) + i), a);
       unpack8e<E>(ld_stream(reinterpret_cast<const uint4*>(g_row) + i), g);
       unpack8e<E>(ld_stream(reinterpret_cast<const uint4*>(g_row + I) + i), u);
+      if constexpr (!ACT) {
+#pragma unroll
+        for (int j = 0; j < 8; j += 2) {
+          a[j] = silu_f32(g[j]), a[j + 1] = silu_f32(g[j + 1]);
+          E::round2(a[j], a[j + 1]);
+          a[j] *= u[j], a[j + 1] *= u[j + 1];
+          E::round2(a[j], a[j + 1]);
+        }
+      }
       float s = 0.f;
 #pragma unroll
       for (int j = 0; j < 8; j += 2) {
@@ -99,7 +109,9 @@ __global__ __launch_bounds__(256) void swiglu_bwd_weighted_kernel(
     for (int64_t j = lane; j < I; j += 64) {
       const float d = E::to_f32(d_row[j]);
       const float dact = E::round(d * w);
-      part += E::round(E::to_f32(a_row[j]) * d);
+      const float a = ACT ? E::to_f32(a_row[j])
+                          : E::round(E::round(silu_f32(E::to_f32(g_row[j]))) * E::to_f32(g_row[I + j]));
+      part += E::round(a * d);
       float dgate, dup;
       swiglu_bwd1<E>(dact, E::to_f32(g_row[j]), E::to_f32(g_row[I + j]), dgate, dup);
       o_row[j] = (bf16_t)E::from_f32(dgate);
@@ -134,23 +146,24 @@ int weight_rows_t(const void* act, const void* row_w, int64_t R, int64_t N, void
   return PMX_OK;
 }
 
-template <class E>
+// ACT false: `act` is not read.
+template <class E, bool ACT>
 int swiglu_bwd_weighted_t(const void* d_act_w, const void* gu, const void* act, const void* row_w,
                             const int32_t* row_src, int64_t R, int64_t I, int64_t A, void* dG1, void* dw,
                             pmx_stream_t stream) {
   if (R < 0 || I < 0 || A < 0) return PMX_ERR_ARG;
   if ((dw == nullptr) != (row_src == nullptr)) return PMX_ERR_ARG;
   if (R == 0) return PMX_OK;
-  if (!row_w || (I > 0 && (!d_act_w || !gu || !act || !dG1))) return PMX_ERR_ARG;
+  if (!row_w || (I > 0 && (!d_act_w || !gu || (ACT && !act) || !dG1))) return PMX_ERR_ARG;
   if ((R + 3) / 4 > (int64_t)INT32_MAX || (I > 0 && R > INT64_MAX / (2 * I))) return PMX_ERR_SHAPE;
   const bool vec = I % 8 == 0 && aligned16(d_act_w) && aligned16(gu) && aligned16(act) && aligned16(dG1);
   const unsigned grid = (unsigned)((R + 3) / 4);
   if (vec)
-    swiglu_bwd_weighted_kernel<E, true><<<grid, 256, 0, stream>>>(
+    swiglu_bwd_weighted_kernel<E, true, ACT><<<grid, 256, 0, stream>>>(
         (const bf16_t*)d_act_w, (const bf16_t*)gu, (const bf16_t*)act, (const bf16_t*)row_w, row_src, R, I, A,
         (bf16_t*)dG1, (bf16_t*)dw);
   else
-    swiglu_bwd_weighted_kernel<E, false><<<grid, 256, 0, stream>>>(
+    swiglu_bwd_weighted_kernel<E, false, ACT><<<grid, 256, 0, stream>>>(
         (const bf16_t*)d_act_w, (const bf16_t*)gu, (const bf16_t*)act, (const bf16_t*)row_w, row_src, R, I, A,
         (bf16_t*)dG1, (bf16_t*)dw);
   PMX_LAUNCH_CHECK();
@@ -173,14 +186,23 @@ int pmx_weight_rows_f16(const void* act, const void* row_w, int64_t R, int64_t N
 int pmx_swiglu_bwd_weighted(const void* d_act_w, const void* gu, const void* act, const void* row_w,
                             const int32_t* row_src, int64_t R, int64_t I, int64_t A, void* dG1, void* dw,
                             pmx_stream_t stream) {
-  return swiglu_bwd_weighted_t<EltBF16>(d_act_w, gu, act, row_w, row_src, R, I, A, dG1, dw, stream);
+  return swiglu_bwd_weighted_t<EltBF16, true>(d_act_w, gu, act, row_w, row_src, R, I, A, dG1, dw, stream);
 }
 
 int pmx_swiglu_bwd_weighted_f16(const void* d_act_w, const void* gu, const void* act, const void* row_w,
                                 const int32_t* row_src, int64_t R, int64_t I, int64_t A, void* dG1, void* dw,
                                 pmx_stream_t stream) {
-  return swiglu_bwd_weighted_t<EltF16>(d_act_w, gu, act, row_w, row_src, R, I, A, dG1, dw, stream);
+  return swiglu_bwd_weighted_t<EltF16, true>(d_act_w, gu, act, row_w, row_src, R, I, A, dG1, dw, stream);
 }
 
+int pmx_swiglu_bwd_weighted_gu(const void* d_act_w, const void* gu, const void* row_w, const int32_t* row_src,
+                               int64_t R, int64_t I, int64_t A, void* dG1, void* dw, pmx_stream_t stream) {
+  return swiglu_bwd_weighted_t<EltBF16, false>(d_act_w, gu, nullptr, row_w, row_src, R, I, A, dG1, dw, stream);
+}
+
+int pmx_swiglu_bwd_weighted_gu_f16(const void* d_act_w, const void* gu, const void* row_w, const int32_t* row_src,
+                                   int64_t R, int64_t I, int64_t A, void* dG1, void* dw, pmx_stream_t stream) {
+  return swiglu_bwd_weighted_t<EltF16, false>(d_act_w, gu, nullptr, row_w, row_src, R, I, A, dG1, dw, stream);
+}
 
 }  // extern "C"

@@ -178,11 +178,12 @@ class _ExpertLayerBase(torch.autograd.Function):
             # group_gemm.py:473-511: fc1_weighted_output = fc1_activation *
             # scattered_gate_weight feeds fc2; moe_gather sums a token's rows.
             xp, row_src, row_w = kernels.moe_scatter_src(hidden, r.pos, routing_weights)
-            gu, act = kernels.gemm_fc1_swiglu(xp, w_gate, w_up, copy_stride, r.offsets, C, inter)
-            act_w = kernels.weight_rows(act, row_w)
+            # the weighted activations straight from the fc1 epilogue; the
+            # backward recomputes the unweighted ones from gu
+            gu, act_w = kernels.gemm_fc1_swiglu(xp, w_gate, w_up, copy_stride, r.offsets, C, inter, row_w=row_w)
             y = kernels.group_gemm_nt(act_w, fc2_weight, r.offsets)
             out = kernels.moe_gather(y, r.pos)
-            ctx.save_for_backward(xp, gu, act, act_w, r.pos, r.offsets, routing_weights, w_gate, w_up, fc2_weight,
+            ctx.save_for_backward(xp, gu, act_w, r.pos, r.offsets, routing_weights, w_gate, w_up, fc2_weight,
                                   row_src, row_w)
             return out
         row_src = None
@@ -250,7 +251,7 @@ class _ExpertLayerBase(torch.autograd.Function):
         """group_gemm.py:533-629: grad_fc2_output = moe_scatter(grad_output);
         its dgrad through fc2, then the router weight's backward with the
         SwiGLU backward in one row kernel; fc1 as in the EP branch."""
-        xp, gu, act, act_w, pos, offsets, w, w_gate, w_up, fc2_weight, row_src, row_w = ctx.saved_tensors
+        xp, gu, act_w, pos, offsets, w, w_gate, w_up, fc2_weight, row_src, row_w = ctx.saved_tensors
         grad_out = grad_out.contiguous()
         need_w, need_x = ctx.needs_input_grad[1], ctx.needs_input_grad[0]
         dyp = kernels.moe_scatter(grad_out, pos)
@@ -262,7 +263,7 @@ class _ExpertLayerBase(torch.autograd.Function):
             with torch.cuda.stream(side):
                 d_fc2 = kernels.group_gemm_tn(dyp, act_w, offsets)
         d_act_w = kernels.group_gemm_nn(dyp, fc2_weight, offsets)
-        dg1, dw = kernels.swiglu_bwd_weighted(d_act_w, gu, act, row_w, row_src, pos.numel())
+        dg1, dw = kernels.swiglu_bwd_weighted(d_act_w, gu, None, row_w, row_src, pos.numel())
         if ctx.fc1_needs_grad:
             side.wait_stream(main)
             with torch.cuda.stream(side):

@@ -292,9 +292,10 @@ def segment_sum(source: torch.Tensor, index: torch.Tensor, num_rows: int) -> tor
 
 
 def gemm_fc1_swiglu(x: torch.Tensor, w_gate: torch.Tensor, w_up: torch.Tensor, copy_stride: int,
-                    offsets: torch.Tensor, num_groups: int, inter: int):
-    """(gu [A,2I], act [A,I]) = SwiGLU fc1 over per-copy row groups."""
-    dev = _check_dev(x, w_gate, w_up, offsets)
+                    offsets: torch.Tensor, num_groups: int, inter: int, row_w: torch.Tensor | None = None):
+    """(gu [A,2I], act [A,I]) = SwiGLU fc1 over per-copy row groups; with the
+    rows' router weights ``row_w`` [A] act is ``weight_rows(act, row_w)``."""
+    dev = _check_dev(x, w_gate, w_up, offsets, row_w)
     dt = _half("hidden", x)
     _half("fc1 gate weight", w_gate, dt)
     _half("fc1 up weight", w_up, dt)
@@ -309,6 +310,14 @@ def gemm_fc1_swiglu(x: torch.Tensor, w_gate: torch.Tensor, w_up: torch.Tensor, c
     )
     gu = torch.empty((A, 2 * inter), dtype=x.dtype, device=dev)
     act = torch.empty((A, inter), dtype=x.dtype, device=dev)
+    if row_w is not None:
+        _half("row weights", row_w, dt)
+        assert row_w.numel() == A, "one router weight per row"
+        _capi.call(
+            _sym("pmx_gemm_fc1_swiglu_weighted_fwd", dt), _ptr(x), _ptr(w_gate), _ptr(w_up), copy_stride,
+            _ptr(offsets), G, A, H, inter, _ptr(row_w), _ptr(gu), _ptr(act), _stream(dev),
+        )
+        return gu, act
     _capi.call(
         _sym("pmx_gemm_fc1_swiglu_fwd", dt), _ptr(x), _ptr(w_gate), _ptr(w_up), int(copy_stride), _ptr(offsets),
         int(num_groups), A, H, int(inter), _ptr(gu), _ptr(act), _stream(dev),
@@ -416,22 +425,29 @@ def weight_rows(act: torch.Tensor, row_w: torch.Tensor) -> torch.Tensor:
     return out
 
 
-def swiglu_bwd_weighted(d_act_w: torch.Tensor, gu: torch.Tensor, act: torch.Tensor, row_w: torch.Tensor,
+def swiglu_bwd_weighted(d_act_w: torch.Tensor, gu: torch.Tensor, act: torch.Tensor | None, row_w: torch.Tensor,
                         row_src: torch.Tensor, num_assign: int):
     """Backward of ``weight_rows`` and the SwiGLU forward, per row:
     dG1 [R, 2I] from dact = bf16(d_act_w * row_w), and the router-weight
     gradient dw[row_src[r]] = bf16(sum_j bf16(act[r,j] * d_act_w[r,j]))
-    -> (dG1, dw [num_assign] bf16; entries no row names are not written)."""
+    -> (dG1, dw [num_assign] bf16; entries no row names are not written).
+    ``act`` None: recomputed from gu (the same bits)."""
     dev = _check_dev(d_act_w, gu, act, row_w, row_src)
-    dt = _half("act", act)
-    for name, t in (("d_act_w", d_act_w), ("gu", gu), ("row weights", row_w)):
+    dt = _half("d_act_w", d_act_w)
+    for name, t in (("gu", gu), ("row weights", row_w)):
         _half(name, t, dt)
-    R, I = act.shape
-    assert d_act_w.shape == (R, I) and gu.shape == (R, 2 * I), "d_act_w [R, I], gu [R, 2I]"
+    R, I = d_act_w.shape
+    assert gu.shape == (R, 2 * I), "d_act_w [R, I], gu [R, 2I]"
     assert row_w.numel() == R and row_w.is_contiguous()
     assert row_src.dtype == torch.int32 and row_src.is_contiguous() and row_src.numel() == R
-    dg1 = torch.empty((R, 2 * I), dtype=act.dtype, device=dev)
+    dg1 = torch.empty((R, 2 * I), dtype=dt, device=dev)
     dw = torch.empty(num_assign, dtype=row_w.dtype, device=dev)
+    if act is None:
+        _capi.call(_sym("pmx_swiglu_bwd_weighted_gu", dt), _ptr(d_act_w), _ptr(gu), _ptr(row_w), _ptr(row_src), R, I,
+                   num_assign, _ptr(dg1), _ptr(dw), _stream(dev))
+        return dg1, dw
+    _half("act", act, dt)
+    assert act.shape == (R, I), "act [R, I]"
     _capi.call(_sym("pmx_swiglu_bwd_weighted", dt), _ptr(d_act_w), _ptr(gu), _ptr(act), _ptr(row_w), _ptr(row_src),
                R, I, num_assign, _ptr(dg1), _ptr(dw), _stream(dev))
     return dg1, dw

@@ -99,3 +99,26 @@ def test_same_as_the_256_row_kernels(cuda, name, dtype):
     torch.cuda.synchronize()
     for k in ref:
         assert_bf16_close(got[k], ref[k], name=f"{name} {k}")
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
+@pytest.mark.parametrize("counts,H,I", [([3, 0, 65, 129], 576, 264), ([300, 1, 0, 257], 512, 192),
+                                        ([1300, 0, 700], 256, 320), ([300, 40], 200, 72)],
+                         ids=["few", "mid", "large", "k_tail"])
+def test_fc1_with_row_weights_is_fc1_then_weight_rows(cuda, counts, H, I, dtype):
+    """Bit for bit, on each kernel that fc1 runs on, and the backward that
+    recomputes the activations against the one that reads them."""
+    off = _off(counts)
+    G, A = len(counts), int(off[-1])
+    offd = torch.as_tensor(off, dtype=torch.int32, device=cuda)
+    gen = torch.Generator(device=cuda).manual_seed(9)
+    rn = lambda *s: torch.randn(s, generator=gen, device=cuda).to(dtype)
+    x, w1, row_w, d = rn(A, H), rn(G, 2 * I, H) * 0.05, rn(A), rn(A, I)
+    up = w1.view(-1)[I * H:]
+    gu, act = kernels.gemm_fc1_swiglu(x, w1, up, 2 * I * H, offd, G, I)
+    gu2, act_w = kernels.gemm_fc1_swiglu(x, w1, up, 2 * I * H, offd, G, I, row_w=row_w)
+    assert torch.equal(gu, gu2) and torch.equal(act_w, kernels.weight_rows(act, row_w))
+    src = torch.randperm(A, generator=gen, device=cuda).to(torch.int32)
+    for got, want in zip(kernels.swiglu_bwd_weighted(d, gu, None, row_w, src, A),
+                         kernels.swiglu_bwd_weighted(d, gu, act, row_w, src, A)):
+        assert torch.equal(got, want)
