@@ -55,7 +55,7 @@ MEASURED_TRAFFIC_BYTES = {
 # Entry-point call order inside one step; repeated names are told apart by
 # their occurrence index.
 STAGES = [
-    ("pmx_route", 0, "route"),
+    ("pmx_route_reported", 0, "route"),
     ("pmx_moe_scatter", 0, "permute"),
     ("pmx_moe_scatter_src", 0, "permute"),
     ("pmx_gemm_fc1_swiglu_fwd", 0, "fc1_fwd"),

@@ -72,6 +72,17 @@ int pmx_route(const int64_t* sel, const int64_t* M, const int64_t* src, int32_t 
               int32_t* phys, int32_t* counts, int32_t* offsets, int32_t* pos,
               void* workspace, size_t workspace_bytes, pmx_stream_t stream);
 
+/* pmx_route that also stores the routing status word to `status_host` (NULL:
+ * not stored): pinned host memory that the device can address, written by the
+ * routing kernel at system scope.  A host that set the word to another value
+ * beforehand can read from it, without waiting, whether the routing has run
+ * and what it found.  The word must stay allocated until then. */
+int pmx_route_reported(const int64_t* sel, const int64_t* M, const int64_t* src, int32_t src_const,
+                       int32_t S, int32_t E, int64_t T, int32_t K, int32_t C,
+                       int32_t* phys, int32_t* counts, int32_t* offsets, int32_t* pos,
+                       void* workspace, size_t workspace_bytes, int32_t* status_host,
+                       pmx_stream_t stream);
+
 /* Allocation-free variant of pmx_route, for callers that cannot allocate
  * (code under HIP graph capture, tight serving loops, harnesses that forbid
  * hipMalloc).  It has no counterpart in the reference.  Same kernels and

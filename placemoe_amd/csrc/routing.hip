@@ -103,6 +103,14 @@ __global__ __launch_bounds__(64) void route_hist_kernel(
   if (lane == 0) flags[ch] = any_bad ? 1 : 0;
 }
 
+// The routing status word, and its copy in pinned host memory (or null),
+// stored at system scope so that the host reads it without a copy behind the
+// routing (a copy kernel and an event: 10 us of the stream per forward).
+__device__ __forceinline__ void put_status(int32_t* status, int32_t* status_host, int32_t v) {
+  status[0] = v;
+  if (status_host != nullptr) __hip_atomic_store(status_host, v, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // Single block: column-wise exclusive scan of the chunk table, turning
 // histogram rows into per-chunk start positions, plus counts, offsets and the
 // status word (the OR of the chunk flags).  With C < 1024 columns the 1024
@@ -113,7 +121,8 @@ __global__ __launch_bounds__(1024) void route_scan_kernel(int32_t* __restrict__ 
                                                           int32_t C, const int32_t* __restrict__ flags,
                                                           int32_t* __restrict__ counts,
                                                           int32_t* __restrict__ offsets,
-                                                          int32_t* __restrict__ status) {
+                                                          int32_t* __restrict__ status,
+                                                          int32_t* __restrict__ status_host) {
   __shared__ int32_t part[1024];  // per (range, column): range sum, then range start
   __shared__ int32_t sums[1024];
   __shared__ int32_t carry_sh;
@@ -206,7 +215,7 @@ __global__ __launch_bounds__(1024) void route_scan_kernel(int32_t* __restrict__ 
       }
     }
   }
-  if (tid == 0) status[0] = bad_sh;
+  if (tid == 0) put_status(status, status_host, bad_sh);
 }
 
 // Assignments of a wave equal to each lane's (bits over the lanes; an invalid
@@ -279,7 +288,7 @@ __global__ __launch_bounds__(64 * kSmallWaves) void route_small_kernel(
     const int64_t* __restrict__ sel, const int64_t* __restrict__ M, const int64_t* __restrict__ src,
     int32_t src_const, int32_t S, int32_t E, int32_t K, int32_t C, int32_t A, int32_t chunk, int nbits,
     int32_t* __restrict__ phys, int32_t* __restrict__ counts, int32_t* __restrict__ offsets,
-    int32_t* __restrict__ pos, int32_t* __restrict__ status) {
+    int32_t* __restrict__ pos, int32_t* __restrict__ status, int32_t* __restrict__ status_host) {
   extern __shared__ int32_t hist[];  // [16][C]: the waves' histograms, then their next positions
   __shared__ int32_t wave_sums[kSmallWaves];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -346,7 +355,7 @@ __global__ __launch_bounds__(64 * kSmallWaves) void route_small_kernel(
   }
   if (tid == 0) {
     offsets[C] = A;
-    status[0] = any_bad ? 1 : 0;
+    put_status(status, status_host, any_bad ? 1 : 0);
   }
   __syncthreads();
   // Stable ranks.  Only this wave touches its row from here on, and a wave's
@@ -383,7 +392,8 @@ inline bool rows_fit(int64_t T, int32_t K) { return T <= INT32_MAX / K; }
 int launch_route(const int64_t* sel, const int64_t* M, const int64_t* src, int32_t src_const,
                  int32_t S, int32_t E, int64_t A, int32_t K, int32_t C, int32_t* phys,
                  int32_t* counts, int32_t* offsets, int32_t* pos, void* workspace,
-                 size_t workspace_bytes, hipStream_t stream, int32_t* status = nullptr) {
+                 size_t workspace_bytes, hipStream_t stream, int32_t* status = nullptr,
+                 int32_t* status_host = nullptr) {
   if (C <= 0 || C > kRouteMaxSlots || A < 0 || K <= 0) return PMX_ERR_ARG;
   if (A > INT32_MAX) return PMX_ERR_SHAPE;  // positions and counts are int32
   if (!counts || !offsets || !workspace) return PMX_ERR_ARG;
@@ -401,7 +411,7 @@ int launch_route(const int64_t* sel, const int64_t* M, const int64_t* src, int32
   if (A > 0 && A <= kSmallMaxAssign && C <= kSmallMaxSlots) {
     const int32_t chunk = (int32_t)((A + 64 * kSmallWaves - 1) / (64 * kSmallWaves)) * 64;
     route_small_kernel<<<1, 64 * kSmallWaves, (size_t)kSmallWaves * C * sizeof(int32_t), stream>>>(
-        sel, M, src, src_const, S, E, K, C, (int32_t)A, chunk, nbits, phys, counts, offsets, pos, status);
+        sel, M, src, src_const, S, E, K, C, (int32_t)A, chunk, nbits, phys, counts, offsets, pos, status, status_host);
     PMX_LAUNCH_CHECK();
     return PMX_OK;
   }
@@ -418,7 +428,7 @@ int launch_route(const int64_t* sel, const int64_t* M, const int64_t* src, int32
         sel, M, src, src_const, S, E, K, C, A, g.chunk, phys, table, flags);
   }
   PMX_LAUNCH_CHECK();
-  route_scan_kernel<<<1, 1024, 0, stream>>>(table, g.nchunks, C, flags, counts, offsets, status);
+  route_scan_kernel<<<1, 1024, 0, stream>>>(table, g.nchunks, C, flags, counts, offsets, status, status_host);
   PMX_LAUNCH_CHECK();
   if (A > 0) {
     if (lds) {
@@ -929,11 +939,19 @@ int pmx_route(const int64_t* sel, const int64_t* M, const int64_t* src, int32_t 
               int32_t E, int64_t T, int32_t K, int32_t C, int32_t* phys, int32_t* counts,
               int32_t* offsets, int32_t* pos, void* workspace, size_t workspace_bytes,
               pmx_stream_t stream) {
+  return pmx_route_reported(sel, M, src, src_const, S, E, T, K, C, phys, counts, offsets, pos, workspace,
+                            workspace_bytes, nullptr, stream);
+}
+
+int pmx_route_reported(const int64_t* sel, const int64_t* M, const int64_t* src, int32_t src_const, int32_t S,
+                       int32_t E, int64_t T, int32_t K, int32_t C, int32_t* phys, int32_t* counts, int32_t* offsets,
+                       int32_t* pos, void* workspace, size_t workspace_bytes, int32_t* status_host,
+                       pmx_stream_t stream) {
   if (T < 0 || K <= 0) return PMX_ERR_ARG;
   if (M == nullptr && src != nullptr) return PMX_ERR_ARG;
   if (T > INT32_MAX / K) return PMX_ERR_SHAPE;
   return launch_route(sel, M, src, src_const, S, E, T * K, K, C, phys, counts, offsets, pos, workspace,
-                      workspace_bytes, stream);
+                      workspace_bytes, stream, nullptr, status_host);
 }
 
 int pmx_route_noalloc(const int64_t* sel, const int64_t* M, const int64_t* src, int32_t src_const, int32_t S,

@@ -33,10 +33,10 @@ import torch
 
 from . import kernels
 
-# Route checks whose status copy has not been looked at yet.  The op never
-# waits for one: each forward and backward polls them (an event query) and
-# raises for the first that has landed and reports an invalid id; a check
-# whose copy is still in flight stays here for the next poll.
+# Route checks whose status has not been looked at yet.  The op never
+# waits for one: each forward and backward polls them (a read of a host word)
+# and raises for the first that has landed and reports an invalid id; a check
+# still in flight stays here for the next poll.
 _PENDING_CHECKS: list = []
 
 
@@ -49,8 +49,8 @@ def _sync_route_checks() -> bool:
 def check_pending_routes(block: bool = False) -> None:
     """Raise ``ValueError`` if a routing call whose status has landed flagged
     an invalid expert or source id.  ``block=True`` first waits for every
-    pending status copy (a host synchronisation: for the end of a step or a
-    test); the default only looks at copies that have already landed."""
+    pending status (a host synchronisation: for the end of a step or a
+    test); the default only looks at those that have already landed."""
     if block:
         for check in _PENDING_CHECKS:
             if not check.checked:
@@ -116,7 +116,7 @@ def _side_stream(device: torch.device) -> torch.cuda.Stream:
 
 
 def _poll_pending_checks() -> None:
-    """Look at every pending check whose copy has landed (no waiting); the
+    """Look at every pending check whose status has landed (no waiting); the
     first that failed raises.  Checks still in flight are kept."""
     keep = []
     failed = None
@@ -158,15 +158,16 @@ class _ExpertLayerBase(torch.autograd.Function):
             f"and hidden size {H} (expected {fc1_shape})"
         )
         _poll_pending_checks()
-        r = kernels.route(selected, C, mapping=mapping, sources=sources, source=source)
         # Invalid expert or source ids are clamped on the device and flagged in
-        # the routing status word.  Its copy is checked without a host sync:
-        # by the backward if it has landed by then, else by a later forward or
-        # backward (or check_pending_routes).
-        check = kernels.RouteCheck(r)
+        # the routing status word, which the routing stores to pinned host
+        # memory.  It is looked at without a host sync: by the backward if it
+        # has landed by then, else by a later forward or backward (or
+        # check_pending_routes).
+        check = kernels.RouteCheck()
+        r = kernels.route(selected, C, mapping=mapping, sources=sources, source=source, check=check)
         if _sync_route_checks():
             check.raise_if_failed()
-        else:
+        elif not check.checked:
             _PENDING_CHECKS.append(check)
         if recorder is not None:
             recorder(r.counts)

@@ -9,6 +9,7 @@ here synchronises the host except ``route_status``.
 from __future__ import annotations
 
 import ctypes
+import threading
 from dataclasses import dataclass
 
 import torch
@@ -25,7 +26,8 @@ def _ptr(t: torch.Tensor | None) -> int | None:
 
 
 def _stream(device: torch.device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    # the handle alone: a torch Stream object costs 4 us, some ten times per forward
+    return torch._C._cuda_getCurrentRawStream(device.index)
 
 
 def _check_dev(*tensors: torch.Tensor | None) -> torch.device:
@@ -81,12 +83,14 @@ def route(
     mapping: torch.Tensor | None = None,
     sources: torch.Tensor | None = None,
     source: int = 0,
+    check: "RouteCheck | None" = None,
 ) -> Routing:
     """phys = mapping[source(t), selected]; counts; offsets; stable scatter index.
 
     ``mapping`` is the source-aware ``M`` table [S, E] (int64 on the device),
     or None for the identity map.  ``sources`` is an int64 [T] per-token source
     id; without it every token uses ``source`` (the reference's ``ep_rank``).
+    The routing reports its status to ``check``.
     """
     dev = _check_dev(selected, mapping, sources)
     sel = selected if selected.dim() == 2 else selected.reshape(-1, 1)
@@ -110,10 +114,17 @@ def route(
     pos = torch.empty((T, K), dtype=torch.int32, device=dev)
     counts = torch.empty(C, dtype=torch.int32, device=dev)
     offsets = torch.empty(C + 1, dtype=torch.int32, device=dev)
-    _capi.call(
-        "pmx_route", _ptr(sel), _ptr(mapping), _ptr(sources), int(source), S, E, T, K, C,
-        _ptr(phys), _ptr(counts), _ptr(offsets), _ptr(pos), _ptr(ws), ws_bytes, _stream(dev),
-    )
+    stream = _stream(dev)
+    status_host = check.arm(dev, stream) if check is not None else None
+    try:
+        _capi.call(
+            "pmx_route_reported", _ptr(sel), _ptr(mapping), _ptr(sources), int(source), S, E, T, K, C,
+            _ptr(phys), _ptr(counts), _ptr(offsets), _ptr(pos), _ptr(ws), ws_bytes, status_host, stream,
+        )
+    except ValueError:  # arguments refused: nothing was launched
+        if check is not None:
+            check.refused()
+        raise
     return Routing(phys=phys, counts=counts, offsets=offsets, pos=pos, workspace=ws)
 
 
@@ -124,25 +135,119 @@ def route_status(r: Routing) -> int:
     return int(out.value)
 
 
-class RouteCheck:
-    """The routing status word, copied to pinned host memory behind the
-    routing kernels on the same stream.  ``ready()`` asks (without waiting)
-    whether the copy has landed; ``failed()`` waits for it."""
+class _StatusWords:
+    """Pinned host words that routing kernels report to.  A word is leased
+    before the launch and given back only once its kernel has written it, so
+    that a late store cannot reach memory that serves another purpose; words
+    whose check was dropped in flight are collected later.  ``BLOCK`` words at
+    a time: more than one block only while more calls than that are in
+    flight."""
 
-    def __init__(self, r: Routing):
-        dev = r.workspace.device
-        self._host = torch.empty(1, dtype=torch.int32, pin_memory=True)
-        self._host.copy_(r.workspace[:4].view(torch.int32), non_blocking=True)
-        self._event = torch.cuda.Event()
-        self._event.record(torch.cuda.current_stream(dev))
+    BLOCK = 4096
+    PENDING = -1
+
+    def __init__(self) -> None:
+        self._lock = threading.Lock()
+        self._blocks: list = []  # (pinned tensor, its address, ctypes view)
+        self._free: list[int] = []
+        self._orphans: list[int] = []
+
+    def _at(self, i: int):
+        return self._blocks[i // self.BLOCK][2], i % self.BLOCK
+
+    def lease(self) -> tuple[int, int]:
+        """(word, its address), the word set to ``PENDING``."""
+        with self._lock:
+            if not self._free:
+                self._collect_orphans()
+            if not self._free:
+                t = torch.empty(self.BLOCK, dtype=torch.int32, pin_memory=True)
+                view = (ctypes.c_int32 * self.BLOCK).from_address(t.data_ptr())
+                self._blocks.append((t, t.data_ptr(), view))
+                n = len(self._blocks) * self.BLOCK
+                self._free = list(range(n - self.BLOCK, n))
+            i = self._free.pop()
+            view, k = self._at(i)
+            view[k] = self.PENDING
+            return i, self._blocks[i // self.BLOCK][1] + 4 * k
+
+    def _collect_orphans(self) -> None:
+        waiting = []
+        for i in self._orphans:
+            view, k = self._at(i)
+            (waiting if view[k] == self.PENDING else self._free).append(i)
+        self._orphans = waiting
+
+    def take(self, check: "RouteCheck") -> None:
+        """Move a landed word's value into its check and free the word."""
+        with self._lock:
+            if check._word is None:
+                return
+            view, k = self._at(check._word)
+            if view[k] != self.PENDING:
+                check._status = int(view[k])
+                self._free.append(check._word)
+                check._word = None
+
+    def give_back(self, i: int) -> None:
+        """A word whose launch was refused."""
+        with self._lock:
+            self._free.append(i)
+
+    def orphan(self, i: int) -> None:
+        """A word whose check is gone while its kernel may still write it."""
+        with self._lock:
+            self._orphans.append(i)
+
+
+_STATUS_WORDS = _StatusWords()
+
+
+class RouteCheck:
+    """The routing status word of one ``route`` call, stored to pinned host
+    memory by the routing kernel itself.  ``ready()`` asks (without waiting)
+    whether it has landed; ``failed()`` waits for it.  A routing captured into
+    a graph reports nothing (every replay would write to the word)."""
+
+    def __init__(self) -> None:
+        self._word: int | None = None
+        self._device: torch.device | None = None
+        self._stream = 0
+        self._status: int | None = None
         self.checked = False
 
+    def arm(self, device: torch.device, stream: int) -> int | None:
+        """The host word's address for a launch on ``stream``."""
+        if torch.cuda.is_current_stream_capturing():
+            self._status, self.checked = 0, True
+            return None
+        self._device, self._stream = device, stream
+        self._word, address = _STATUS_WORDS.lease()
+        return address
+
+    def refused(self) -> None:
+        """The launch was refused before anything ran."""
+        if self._word is not None:
+            _STATUS_WORDS.give_back(self._word)
+            self._word = None
+
     def ready(self) -> bool:
-        return self._event.query()
+        if self._status is None:
+            _STATUS_WORDS.take(self)
+        return self._status is not None
 
     def failed(self) -> bool:
-        self._event.synchronize()
-        return int(self._host[0]) != 0
+        if not self.ready():
+            stream = (torch.cuda.ExternalStream(self._stream, device=self._device) if self._stream
+                      else torch.cuda.default_stream(self._device))
+            stream.synchronize()
+            if not self.ready():
+                raise RuntimeError("the routing kernel has run without reporting its status")
+        return self._status != 0
+
+    def __del__(self) -> None:
+        if self._word is not None:
+            _STATUS_WORDS.orphan(self._word)
 
     def raise_if_failed(self) -> None:
         self.checked = True
