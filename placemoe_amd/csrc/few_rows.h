@@ -470,4 +470,116 @@ __global__ __launch_bounds__(CF::NT, CF::NW * CF::BPC / 4) void few_rows_grouped
   wait_loads<0>();
 }
 
+// Weight gradient of copies with few rows: C[g] = A[rows g]^T B[rows g] with
+// one or two 64-row K-tiles, bound by writing C.  The persistent 256 x 256
+// kernel spends a tile there on one K-tile and then on an epilogue during
+// which the CU does nothing else; here a block computes one 128 x 128 tile
+// (4 waves of 64 x 64, 32 KB of LDS, four blocks per CU), so that the blocks
+// of a CU load, multiply and store beside each other.  Operands, both
+// [64 k][128] in LDS, and fragments as in the other kernels; the output goes
+// through the same LDS and leaves as whole 128-byte row pieces.
+constexpr int kWgT = 128, kWgNT = 256;
+
+__global__ __launch_bounds__(kWgNT, 4) void few_rows_wgrad_grouped_gemm_kernel(GemmParams P) {
+  constexpr int QL = 4;  // 1 KB loads per wave and operand
+  __shared__ __attribute__((aligned(1024))) char lds[2 * kWgT * BK * 2];
+  char* As = lds;
+  char* Bs = lds + kWgT * BK * 2;
+  const int lane = threadIdx.x & 63;
+  const int wave = uni(threadIdx.x >> 6);
+  const int wm = wave >> 1, wn = wave & 1;
+
+  // Each XCD (blocks go round-robin over them) takes its own eighth of the
+  // tiles, copy by copy, n fastest.
+  const int64_t ntn = (P.N + kWgT - 1) / kWgT, per_g = (P.M + kWgT - 1) / kWgT * ntn;
+  const int64_t total = per_g * P.G, per_x = gridDim.x / kNumXcd;
+  const int64_t tile = (int64_t)(blockIdx.x % kNumXcd) * per_x + blockIdx.x / kNumXcd;
+  if (tile >= total) return;
+  const int64_t g = tile / per_g, m0 = (tile - g * per_g) / ntn * kWgT, n0 = (tile - g * per_g) % ntn * kWgT;
+  const int64_t row0 = P.offsets[g], row_end = P.offsets[g + 1];
+
+  f32x4_t acc[4][4];
+#pragma unroll
+  for (int m = 0; m < 4; ++m)
+#pragma unroll
+    for (int n = 0; n < 4; ++n) acc[m][n] = f32x4_t{};
+
+  // Load q covers k-rows 4q .. 4q+3, lane i k-row 4q + i/16, physical chunk
+  // i%16 = logical chunk ^ mn_swz; k-rows past the copy fail the range check.
+  uint32_t oa[QL], ob[QL];
+#pragma unroll
+  for (int q = 0; q < QL; ++q) {
+    const int krow = (q * 4 + wave) * 4 + (lane >> 4);
+    const int c = (lane & 15) ^ w4::mn_swz(krow);
+    oa[q] = m0 + c * 8 < P.M ? (uint32_t)(krow * P.a.ld * 2 + (m0 + c * 8) * 2) : kOOB;
+    ob[q] = n0 + c * 8 < P.N ? (uint32_t)(krow * P.b.ld * 2 + (n0 + c * 8) * 2) : kOOB;
+  }
+  const int gq = lane >> 4, i16 = lane & 15;
+  const int base = (gq * 8 + (i16 >> 2)) * (2 * kWgT) + (i16 & 1) * 8;
+  const int sw = w4::mn_swz(gq * 8 + (i16 >> 2));
+  auto frag = [&](const char* t, int cb, int ks) __attribute__((always_inline)) {
+    const char* p = t + ks * 32 * (2 * kWgT) + base + ((((cb >> 3) + ((i16 & 3) >> 1)) ^ sw) << 4);
+    const bf16x4_t v0 = __builtin_amdgcn_ds_read_tr16_b64_v4bf16(LDS_TR_PTR(p));
+    const bf16x4_t v1 = __builtin_amdgcn_ds_read_tr16_b64_v4bf16(LDS_TR_PTR(p + 4 * (2 * kWgT)));
+    return bf16x8_t{v0[0], v0[1], v0[2], v0[3], v1[0], v1[1], v1[2], v1[3]};
+  };
+  for (int64_t r = row0; r < row_end; r += BK) {
+    const int64_t rows = uni64(row_end - r < BK ? row_end - r : BK);
+    const __amdgpu_buffer_rsrc_t ra = make_rsrc(P.a.p0 + uni64(r) * P.a.ld, (uint64_t)rows * P.a.ld * 2);
+    const __amdgpu_buffer_rsrc_t rb = make_rsrc(P.b.p0 + uni64(r) * P.b.ld, (uint64_t)rows * P.b.ld * 2);
+#pragma unroll
+    for (int q = 0; q < QL; ++q) {
+      dma16(ra, As + (q * 4 + wave) * 1024, oa[q], 0);
+      dma16(rb, Bs + (q * 4 + wave) * 1024, ob[q], 0);
+    }
+    wait_loads<0>();
+    block_barrier();
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) {
+      if (ks * 32 >= rows) break;
+      bf16x8_t a[4], b[4];
+#pragma unroll
+      for (int m = 0; m < 4; ++m) a[m] = frag(As, wm * 64 + m * 16, ks);
+#pragma unroll
+      for (int n = 0; n < 4; ++n) b[n] = frag(Bs, wn * 64 + n * 16, ks);
+#pragma unroll
+      for (int m = 0; m < 4; ++m)
+#pragma unroll
+        for (int n = 0; n < 4; ++n) acc[m][n] = mfma16(b[n], a[m], acc[m][n]);
+    }
+    wait_lds();
+    block_barrier();  // every wave has read the stage
+  }
+
+  // The wave's 64 x 64 tile through its own 8 KB: row r at 128 bytes, 16-byte
+  // chunk c at c ^ ((r >> 1) & 7); then 8 rows x 128 bytes per store.
+  char* st = lds + wave * 8192;
+  const int h = lane >> 4;
+#pragma unroll
+  for (int m = 0; m < 4; ++m)
+#pragma unroll
+    for (int n = 0; n < 4; ++n) {
+      const int r = m * 16 + (lane & 15), x = n * 32 + h * 8;
+      *reinterpret_cast<uint2*>(st + r * 128 + (((x >> 4) ^ kc_swz(r)) << 4) + (x & 15)) = w4::bf16x4(acc[m][n]);
+    }
+  wait_lds();
+  const int64_t col = n0 + wn * 64 + (lane & 7) * 8;
+  const bool whole_lines = P.ldc % 64 == 0;
+#pragma unroll
+  for (int q = 0; q < 8; ++q) {
+    const int r = q * 8 + (lane >> 3);
+    const uint4 v = *reinterpret_cast<const uint4*>(st + r * 128 + (((lane & 7) ^ kc_swz(r)) << 4));
+    const int64_t m = m0 + wm * 64 + r;
+    if (m < P.M && col < P.N) {
+      bf16_t* crow = m < P.csplit ? P.c0 + g * P.cgs + m * P.ldc : P.c1 + g * P.cgs + (m - P.csplit) * P.ldc;
+      // Streaming stores of whole lines; rows off the 128-byte lines leave
+      // partial ones, which the L2 must merge before they go to memory (fc2
+      // wgrad of 40 copies of 2048 x 1416: 48 us with plain stores, 107 with
+      // streaming ones; of 160 of 2048 x 768, whole lines: 115 and 86).
+      if (whole_lines) st_stream(crow + col, v);
+      else *reinterpret_cast<uint4*>(crow + col) = v;
+    }
+  }
+}
+
 }  // namespace fr

@@ -122,3 +122,30 @@ def test_fc1_with_row_weights_is_fc1_then_weight_rows(cuda, counts, H, I, dtype)
     for got, want in zip(kernels.swiglu_bwd_weighted(d, gu, None, row_w, src, A),
                          kernels.swiglu_bwd_weighted(d, gu, act, row_w, src, A)):
         assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
+@pytest.mark.parametrize("split", [False, True])
+@pytest.mark.parametrize("counts,M,N", [([1, 0, 31, 32, 33, 63, 64, 65, 0, 129], 264, 136), ([128], 128, 128),
+                                        ([0, 0, 0, 5], 8, 1024), ([200, 0, 56], 400, 72), ([90] * 20, 136, 200)])
+def test_weight_gradient(cuda, counts, M, N, split, dtype):
+    """Few rows per copy: against fp32 products and the 256-row kernels; empty
+    copies are zero, rows past the last copy (NaN here) reach nothing."""
+    off = _off(counts)
+    G, A = len(counts), int(off[-1])
+    offd = torch.as_tensor(off, dtype=torch.int32, device=cuda)
+    gen = torch.Generator(device=cuda).manual_seed(M + N)
+    a = torch.randn((A + 70, M), generator=gen, device=cuda).to(dtype)
+    b = torch.randn((A + 70, N), generator=gen, device=cuda).to(dtype)
+    a[A:] = float("nan")
+    b[A:] = float("nan")
+    run = lambda: kernels.group_gemm_tn(a, b, offd, split=M // 2 if split else None)
+    got = run()
+    with _capi.using(build.variant_path("w8")):
+        ref = run()
+    got, ref = (torch.cat(t, 1) if split else t for t in (got, ref))
+    assert_bf16_close(got, ref, name="against the 256-row kernel")
+    for g, n in enumerate(counts):
+        s = int(off[g])
+        want = a[s:s + n].float().t() @ b[s:s + n].float() if n else torch.zeros((M, N), device=cuda)
+        assert_bf16_close(got[g], want, name=f"copy {g} ({n} rows)")
