@@ -10,6 +10,7 @@ from __future__ import annotations
 
 import ctypes
 import threading
+from collections import deque
 from dataclasses import dataclass
 
 import torch
@@ -150,7 +151,7 @@ class _StatusWords:
         self._lock = threading.Lock()
         self._blocks: list = []  # (pinned tensor, its address, ctypes view)
         self._free: list[int] = []
-        self._orphans: list[int] = []
+        self._orphans: deque = deque()
 
     def _at(self, i: int):
         return self._blocks[i // self.BLOCK][2], i % self.BLOCK
@@ -172,11 +173,10 @@ class _StatusWords:
             return i, self._blocks[i // self.BLOCK][1] + 4 * k
 
     def _collect_orphans(self) -> None:
-        waiting = []
-        for i in self._orphans:
+        for _ in range(len(self._orphans)):
+            i = self._orphans.popleft()
             view, k = self._at(i)
-            (waiting if view[k] == self.PENDING else self._free).append(i)
-        self._orphans = waiting
+            (self._orphans if view[k] == self.PENDING else self._free).append(i)
 
     def take(self, check: "RouteCheck") -> None:
         """Move a landed word's value into its check and free the word."""
@@ -195,9 +195,10 @@ class _StatusWords:
             self._free.append(i)
 
     def orphan(self, i: int) -> None:
-        """A word whose check is gone while its kernel may still write it."""
-        with self._lock:
-            self._orphans.append(i)
+        """A word whose check is gone while its kernel may still write it.
+        Without the lock: a garbage collection can end a check, and so come
+        here, on a thread that holds it (``deque.append`` is atomic)."""
+        self._orphans.append(i)
 
 
 _STATUS_WORDS = _StatusWords()
