@@ -290,7 +290,10 @@ class LayerPlacement:
         if self.accumulated_slot_tokens is None or self.accumulated_slot_tokens.shape != counts.shape:
             self.accumulated_slot_tokens = counts.to(torch.int64, copy=True)
         else:
-            self.accumulated_slot_tokens.add_(counts)  # int32 counts into the int64 sums: one kernel
+            # int32 counts (the routing's) into the int64 sums in one kernel;
+            # types that int64 does not take in place are converted first
+            integer = counts.dtype in (torch.int32, torch.int64)
+            self.accumulated_slot_tokens.add_(counts if integer else counts.to(torch.int64))
 
     def clear_slot_tokens(self) -> None:
         self.accumulated_slot_tokens = None

@@ -113,3 +113,13 @@ def test_slot_token_accumulation():
     assert lp.accumulated_slot_tokens.tolist() == [2, 1, 2, 0, 0, 3]
     lp.clear_slot_tokens()
     assert lp.accumulated_slot_tokens is None
+
+
+@pytest.mark.parametrize("dtype", [torch.int32, torch.int64, torch.int16, torch.float32, torch.bool])
+def test_slot_tokens_of_any_count_type(dtype):
+    lp = LayerPlacement.from_plan("l0", PLAN, num_experts=4)
+    counts = torch.tensor([1, 0, 1, 1, 0, 1], dtype=dtype)
+    lp.record_slot_tokens(counts)
+    lp.record_slot_tokens(counts)
+    assert lp.accumulated_slot_tokens.dtype == torch.int64
+    assert lp.accumulated_slot_tokens.tolist() == [2, 0, 2, 2, 0, 2]
