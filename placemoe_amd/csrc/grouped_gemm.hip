@@ -2323,13 +2323,15 @@ int launch(const GemmParams& P, hipStream_t stream) {
     const bool fast = P.K % BK == 0 && (KIND != KIND_NN || P.b.split >= P.K);
     // fc1 with up to kRsFc1Rows rows per copy: the register-staged loads, with
     // two K-tiles to land, as for fc2 and the fc1 dgrad (us, register-staged /
-    // four-wave: 128 copies of 256 rows of 2048 x 768 302 / 325, 400 rows 404 /
-    // 414-444, 32 copies of 500 rows of 4096 x 1536 421-430 / 428-437; past it
-    // the four-wave kernel: 160 copies of 819 rows 856-870 / 824-861).
+    // four-wave: 128 copies of 256 rows of 2048 x 768 302 / 325).  Above it the
+    // four-wave kernel: at 400-500 rows it takes 1-6% longer by itself (400
+    // rows 414-444 / 404), but its loads draw less power, and the GEMMs that
+    // follow run 2% faster (256 copies of 512 rows, training step with fold:
+    // 6077 us against 6216 with the register-staged fc1).
     // Row weights (non-EP) too: the four-wave epilogue has no register left for
     // them (2 spill), and a separate pass over act costs more than the 1-3%
     // between the kernels.
-    constexpr int64_t kRsFc1Rows = 600;
+    constexpr int64_t kRsFc1Rows = 320;
     [[maybe_unused]] const bool rs_fc1 = KIND == KIND_FC1 && (P.row_w != nullptr || P.M <= kRsFc1Rows * P.G);
     if constexpr (use_w4<KIND>()) {
       if (fast && !rs_fc1) {
