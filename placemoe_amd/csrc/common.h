@@ -183,13 +183,25 @@ __device__ __forceinline__ float wave_sum(float v) {
 
 static inline int pmx_status(hipError_t e) { return e == hipSuccess ? PMX_OK : PMX_ERR_HIP; }
 
-// The routing path's stable counting sort (routing.hip), shared with the
+// Lanes of the wave that hold the same value as this one (the low `nbits`
+// bits of v; an invalid lane equals nothing).
+__device__ __forceinline__ uint64_t match_any(int32_t v, bool valid, int nbits) {
+  uint64_t mask = __ballot(valid);
+  for (int b = 0; b < nbits; ++b) {
+    const bool bit = (v >> b) & 1;
+    const uint64_t m = __ballot(bit);
+    mask &= bit ? m : ~m;
+  }
+  return mask;
+}
+
+// The scan of the routing path's counting sort (routing.hip), shared with the
 // expert-parallel payload builder (payload.hip); not part of the C ABI.
-__attribute__((visibility("hidden"))) int pmx_route_launch(
-    const int64_t* sel, const int64_t* M, const int64_t* src, int32_t src_const, int32_t S, int32_t E, int64_t A,
-    int32_t K, int32_t C, int32_t* phys, int32_t* counts, int32_t* offsets, int32_t* pos, void* workspace,
-    size_t workspace_bytes, hipStream_t stream);
-__attribute__((visibility("hidden"))) size_t pmx_route_ws_bytes(int64_t A, int32_t C);
+// table [nchunks][C]: counts per chunk and column -> start positions; counts
+// [C], offsets [C + 1]; *status = any of flags [nchunks].
+__attribute__((visibility("hidden"))) int pmx_route_scan_launch(int32_t* table, int64_t nchunks, int32_t C,
+                                                                const int32_t* flags, int32_t* counts,
+                                                                int32_t* offsets, int32_t* status, hipStream_t stream);
 
 #define PMX_LAUNCH_CHECK()                         \
   do {                                             \

@@ -218,18 +218,6 @@ __global__ __launch_bounds__(1024) void route_scan_kernel(int32_t* __restrict__ 
   if (tid == 0) put_status(status, status_host, bad_sh);
 }
 
-// Assignments of a wave equal to each lane's (bits over the lanes; an invalid
-// lane equals nothing).
-__device__ __forceinline__ uint64_t match_any(int32_t v, bool valid, int nbits) {
-  uint64_t mask = __ballot(valid);
-  for (int b = 0; b < nbits; ++b) {
-    const bool bit = (v >> b) & 1;
-    const uint64_t m = __ballot(bit);
-    mask &= bit ? m : ~m;
-  }
-  return mask;
-}
-
 // One wave per chunk: stable rank of every assignment among equal copies.
 template <bool USE_LDS>
 __global__ __launch_bounds__(64) void route_rank_kernel(const int32_t* __restrict__ phys,
@@ -872,14 +860,12 @@ inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 
 
 }  // namespace
 
-int pmx_route_launch(const int64_t* sel, const int64_t* M, const int64_t* src, int32_t src_const, int32_t S,
-                     int32_t E, int64_t A, int32_t K, int32_t C, int32_t* phys, int32_t* counts, int32_t* offsets,
-                     int32_t* pos, void* workspace, size_t workspace_bytes, hipStream_t stream) {
-  return launch_route(sel, M, src, src_const, S, E, A, K, C, phys, counts, offsets, pos, workspace, workspace_bytes,
-                      stream);
+int pmx_route_scan_launch(int32_t* table, int64_t nchunks, int32_t C, const int32_t* flags, int32_t* counts,
+                          int32_t* offsets, int32_t* status, hipStream_t stream) {
+  route_scan_kernel<<<1, 1024, 0, stream>>>(table, nchunks, C, flags, counts, offsets, status, nullptr);
+  PMX_LAUNCH_CHECK();
+  return PMX_OK;
 }
-
-size_t pmx_route_ws_bytes(int64_t A, int32_t C) { return route_ws_bytes(A, C); }
 
 // ---------------------------------------------------------------------------
 // Device scratch of pmx_route_noalloc: the routing chunk table lives in a

@@ -63,16 +63,16 @@ def build_local_payload(hidden_states: torch.Tensor, selected_experts: torch.Ten
     Hp = H + pad
 
     i32 = dict(dtype=torch.int32, device=device)
-    assign_counts = torch.empty(ep_size, **i32)
+    # one buffer for what the host reads: assignment and row counts per rank, status
+    host_counts = torch.zeros(2 * ep_size + 1, **i32)
+    assign_counts, unique_counts, status = host_counts.split([ep_size, ep_size, 1])
     assign_offsets = torch.empty(ep_size + 1, **i32)
-    unique_counts = torch.empty(ep_size, **i32)
     unique_offsets = torch.empty(ep_size + 1, **i32)
     send_hidden = torch.empty((A, Hp), dtype=dt, device=device)
     unique_tokens = torch.empty(A, **i32)
     send_meta = torch.empty((A, 3), **i32)
     send_weights = torch.empty(A, dtype=dt, device=device)
     target_rank = torch.empty(A, **i32)
-    status = torch.zeros(1, **i32)
     ws = _workspace(_capi.load().pmx_ep_payload_workspace_bytes(A, ep_size), device)
     _capi.call(
         "pmx_ep_dispatch_payload", phys.data_ptr() if A else None, hidden.data_ptr() if T else None,
@@ -82,7 +82,7 @@ def build_local_payload(hidden_states: torch.Tensor, selected_experts: torch.Ten
         send_meta.data_ptr() if A else None, send_weights.data_ptr() if A else None,
         target_rank.data_ptr() if A else None, status.data_ptr(), ws.data_ptr(), ws.numel(), _stream(device),
     )
-    counts = torch.cat([assign_counts, unique_counts, status]).cpu().tolist()
+    counts = host_counts.cpu().tolist()
     if counts[-1]:
         raise ValueError("physical expert id outside [0, num_experts)")
     assignment_send_splits = [int(c) for c in counts[:ep_size]]
@@ -123,9 +123,8 @@ def combine_aggregate(expert_outputs: torch.Tensor, pos: torch.Tensor, recv_weig
     tokens = source_token_indices.to(**i32).contiguous()
     out = torch.empty((max(N, 1), Hp), dtype=dt, device=device)
     run_offsets = torch.empty(N + 1, **i32)
-    rank_runs = torch.empty(ep_size, **i32)
-    num_runs = torch.empty(1, **i32)
-    status = torch.zeros(1, **i32)
+    host_counts = torch.zeros(ep_size + 2, **i32)
+    rank_runs, num_runs, status = host_counts.split([ep_size, 1, 1])
     ws = _workspace(_capi.load().pmx_ep_combine_workspace_bytes(N), device)
     name = "pmx_ep_combine_aggregate_f16" if dt == torch.float16 else "pmx_ep_combine_aggregate"
     _capi.call(
@@ -134,7 +133,7 @@ def combine_aggregate(expert_outputs: torch.Tensor, pos: torch.Tensor, recv_weig
         run_offsets.data_ptr(), rank_runs.data_ptr(), num_runs.data_ptr(), status.data_ptr(), ws.data_ptr(),
         ws.numel(), _stream(device),
     )
-    host = torch.cat([rank_runs, num_runs, status]).cpu().tolist()
+    host = host_counts.cpu().tolist()
     if host[-1]:
         raise ValueError("source rank outside [0, ep_size)")
     U = int(host[ep_size])

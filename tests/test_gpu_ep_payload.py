@@ -112,3 +112,39 @@ def test_round_trip_across_simulated_ranks(cuda, seed, R, L, T, K, H):
             for k in range(K):
                 eager[t] += w[r][t, k].double() * (hid[r][t].double() @ W[phys[r][t, k]].double().t())
         assert_bf16_close(outs[r].cpu().to(torch.bfloat16), eager.float())
+
+
+# Segments of whole tokens (64 // K of them), chunks of four segments, more
+# than 1024 chunks, one rank, and more ranks than LDS counters (4096).
+@pytest.mark.parametrize("T,K,R,L", [(1, 1, 1, 1), (63, 1, 3, 2), (257, 1, 2, 1), (36, 7, 4, 3), (37, 7, 4, 3),
+                                     (9, 22, 5, 4), (8, 32, 2, 9), (40001, 7, 8, 2), (90, 6, 4096, 1),
+                                     (90, 6, 4097, 1), (700, 3, 5000, 2)])
+def test_payload_at_segment_and_chunk_edges(cuda, T, K, R, L):
+    print(f"payload T={T} K={K} R={R} L={L}", flush=True)
+    g = torch.Generator().manual_seed(T + K)
+    phys = torch.randint(0, R * L, (T, K), generator=g)
+    phys[::3] = phys[::3] % max(1, R * L // 3)  # several assignments of a token on one rank
+    phys[1::5] = R * L - 1  # ... and all of them
+    hidden = torch.randn(T, 8, generator=g).to(torch.bfloat16)
+    w = torch.rand(T, K, generator=g).to(torch.bfloat16)
+    _check_payload(cuda, hidden, phys.numpy(), w, R * L, R)
+
+
+# Runs past 64 rows, odd ones, and rows around the 64 and 256 chunks of a pass.
+@pytest.mark.parametrize("H", [8, 504, 520, 2040, 2048, 2056, 4104])
+def test_combine_aggregate_run_lengths(cuda, H):
+    g = torch.Generator().manual_seed(H)
+    lengths = [1, 2, 3, 63, 64, 65, 1, 128, 129, 200, 5]
+    tokens = np.repeat(np.arange(len(lengths)), lengths)
+    N = len(tokens)
+    splits = [int(sum(lengths[:4])), 0, int(sum(lengths[4:]))]
+    y = torch.randn(N, H, generator=g).to(torch.bfloat16)
+    pos = torch.randperm(N, generator=g)
+    w = torch.rand(N, generator=g).to(torch.bfloat16)
+    ranks = torch.repeat_interleave(torch.arange(3), torch.as_tensor(splits))
+    got, gsplits = EP.combine_aggregate(y.to(cuda), pos.to(cuda), w.to(cuda), ranks.to(cuda),
+                                        torch.as_tensor(tokens).to(cuda), 3)
+    weighted = (y[pos].float() * w.float()[:, None]).to(torch.bfloat16)
+    ref, rsplits = O.aggregate_weighted_outputs(weighted, tokens, splits)
+    assert gsplits == rsplits
+    assert_bf16_close(got.cpu(), ref)
