@@ -421,6 +421,15 @@ int pmx_ep_dispatch_payload(const int32_t* phys, const void* hidden, const void*
                             int32_t* send_meta, void* send_weights, int32_t* target_rank,
                             int32_t* status, void* workspace, size_t workspace_bytes,
                             pmx_stream_t stream);
+/* The same with int64 phys, unique_tokens and target_rank (the types of the
+ * reference's tensors); the low 32 bits of a slot count. */
+int pmx_ep_dispatch_payload_i64(const int64_t* phys, const void* hidden, const void* weights, int64_t T,
+                            int32_t K, int64_t H, int32_t R, int32_t slots_per_rank,
+                            int32_t* assign_counts, int32_t* assign_offsets, int32_t* unique_counts,
+                            int32_t* unique_offsets, void* send_hidden, int64_t* unique_tokens,
+                            int32_t* send_meta, void* send_weights, int64_t* target_rank,
+                            int32_t* status, void* workspace, size_t workspace_bytes,
+                            pmx_stream_t stream);
 
 /* Bytes of workspace pmx_ep_combine_aggregate needs for `num_recv` received
  * assignments. */
@@ -440,6 +449,12 @@ size_t pmx_ep_combine_workspace_bytes(int64_t num_recv);
  * 2266-2294). */
 int pmx_ep_combine_aggregate(const void* Y, const int32_t* pos, const void* w, const int32_t* src_rank,
                              const int32_t* src_token, int64_t N, int64_t H, int32_t R, void* out,
+                             int32_t* run_offsets, int32_t* rank_runs, int32_t* num_runs,
+                             int32_t* status, void* workspace, size_t workspace_bytes,
+                             pmx_stream_t stream);
+/* The same with int64 pos, src_rank and src_token; the low 32 bits count. */
+int pmx_ep_combine_aggregate_i64(const void* Y, const int64_t* pos, const void* w, const int64_t* src_rank,
+                             const int64_t* src_token, int64_t N, int64_t H, int32_t R, void* out,
                              int32_t* run_offsets, int32_t* rank_runs, int32_t* num_runs,
                              int32_t* status, void* workspace, size_t workspace_bytes,
                              pmx_stream_t stream);
@@ -505,6 +520,11 @@ int pmx_replica_fold_f16(void* grads, const int32_t* copy_offsets, const int32_t
                          int32_t writeback, int32_t* status, pmx_stream_t stream);
 int pmx_ep_combine_aggregate_f16(const void* Y, const int32_t* pos, const void* w, const int32_t* src_rank,
                                  const int32_t* src_token, int64_t N, int64_t H, int32_t R, void* out,
+                                 int32_t* run_offsets, int32_t* rank_runs, int32_t* num_runs,
+                                 int32_t* status, void* workspace, size_t workspace_bytes,
+                                 pmx_stream_t stream);
+int pmx_ep_combine_aggregate_i64_f16(const void* Y, const int64_t* pos, const void* w, const int64_t* src_rank,
+                                 const int64_t* src_token, int64_t N, int64_t H, int32_t R, void* out,
                                  int32_t* run_offsets, int32_t* rank_runs, int32_t* num_runs,
                                  int32_t* status, void* workspace, size_t workspace_bytes,
                                  pmx_stream_t stream);

@@ -82,10 +82,12 @@ __device__ __forceinline__ Peers peers(int32_t r, bool valid, int nbits, int lan
 
 // Per chunk: target ranks, and the counts of the chunk's assignments (columns
 // 0 .. R-1 of its table row) and of its (rank, token) pairs (R .. 2R-1) per rank.
-template <bool USE_LDS>
-__global__ __launch_bounds__(64) void payload_hist_kernel(const int32_t* __restrict__ phys, int64_t A, int32_t K,
+// (I: the index type of the caller's slots, ranks and tokens, of which the low
+// 32 bits count.)
+template <bool USE_LDS, class I>
+__global__ __launch_bounds__(64) void payload_hist_kernel(const I* __restrict__ phys, int64_t A, int32_t K,
                                                           int32_t R, int32_t L, int32_t seg, int64_t chunk, int nbits,
-                                                          int32_t* __restrict__ target_rank,
+                                                          I* __restrict__ target_rank,
                                                           int32_t* __restrict__ table, int32_t* __restrict__ flags,
                                                           int32_t* __restrict__ status) {
   extern __shared__ int32_t lds_hist[];
@@ -103,7 +105,7 @@ __global__ __launch_bounds__(64) void payload_hist_kernel(const int32_t* __restr
 #pragma unroll
     for (int u = 0; u < kPayloadSegs; ++u) {
       const int64_t a = s + u * seg + lane;
-      p[u] = lane < seg && a < end ? phys[a] : 0;
+      p[u] = lane < seg && a < end ? (int32_t)phys[a] : 0;
     }
 #pragma unroll
     for (int u = 0; u < kPayloadSegs; ++u) {
@@ -133,13 +135,13 @@ __global__ __launch_bounds__(64) void payload_hist_kernel(const int32_t* __restr
 // its row (upos; -1 at the others).  `table` holds the chunks' start
 // positions, those of the pairs behind the A assignments.  Block 0 writes the
 // counts and offsets out.
-template <bool USE_LDS>
+template <bool USE_LDS, class I>
 __global__ __launch_bounds__(64) void payload_place_kernel(
-    const int32_t* __restrict__ phys, const bf16_t* __restrict__ weights, int64_t A, int32_t K, int32_t R, int32_t L,
+    const I* __restrict__ phys, const bf16_t* __restrict__ weights, int64_t A, int32_t K, int32_t R, int32_t L,
     int32_t seg, int64_t chunk, int nbits, int32_t* __restrict__ table, const int32_t* __restrict__ counts,
     const int32_t* __restrict__ offsets, int32_t* __restrict__ assign_counts, int32_t* __restrict__ assign_offsets,
     int32_t* __restrict__ unique_counts, int32_t* __restrict__ unique_offsets, int32_t* __restrict__ send_meta,
-    bf16_t* __restrict__ send_weights, int32_t* __restrict__ unique_tokens, int32_t* __restrict__ upos) {
+    bf16_t* __restrict__ send_weights, I* __restrict__ unique_tokens, int32_t* __restrict__ upos) {
   extern __shared__ int32_t lds_pos[];
   const int lane = threadIdx.x;
   if (blockIdx.x == 0) {
@@ -169,7 +171,7 @@ __global__ __launch_bounds__(64) void payload_place_kernel(
     for (int u = 0; u < kPayloadSegs; ++u) {
       const int64_t a = s + u * seg + lane;
       const bool valid = lane < seg && a < end;
-      p[u] = valid ? phys[a] : 0;
+      p[u] = valid ? (int32_t)phys[a] : 0;
       w[u] = valid ? weights[a] : (bf16_t)0;
     }
 #pragma unroll
@@ -251,8 +253,9 @@ constexpr int kScanBlock = 1024;
 
 // flag[a] = 1 where a run of equal (src_rank, src_token) starts; per-block
 // sums of the flags; rank_runs cleared for the counts that follow.
-__global__ __launch_bounds__(kScanBlock) void run_flags_kernel(const int32_t* __restrict__ src_rank,
-                                                               const int32_t* __restrict__ src_token, int64_t N,
+template <class I>
+__global__ __launch_bounds__(kScanBlock) void run_flags_kernel(const I* __restrict__ src_rank,
+                                                               const I* __restrict__ src_token, int64_t N,
                                                                int32_t* __restrict__ flag,
                                                                int32_t R, int32_t* __restrict__ rank_runs,
                                                                int32_t* __restrict__ block_sum) {
@@ -261,7 +264,10 @@ __global__ __launch_bounds__(kScanBlock) void run_flags_kernel(const int32_t* __
   for (int64_t r = a; r < R; r += (int64_t)gridDim.x * kScanBlock) rank_runs[r] = 0;
   int32_t f = 0;
   if (a < N) {
-    f = (a == 0 || src_rank[a] != src_rank[a - 1] || src_token[a] != src_token[a - 1]) ? 1 : 0;
+    f = (a == 0 || (int32_t)src_rank[a] != (int32_t)src_rank[a - 1] ||
+         (int32_t)src_token[a] != (int32_t)src_token[a - 1])
+            ? 1
+            : 0;
     flag[a] = f;
   }
   const uint64_t m = __ballot(f != 0);
@@ -308,9 +314,10 @@ __global__ __launch_bounds__(kScanBlock) void scan_blocks_kernel(int32_t* __rest
 // R counters.
 constexpr int kLdsRanks = 4096;
 
+template <class I>
 __global__ __launch_bounds__(kScanBlock) void run_offsets_kernel(const int32_t* __restrict__ flag,
                                                                  const int32_t* __restrict__ block_base,
-                                                                 const int32_t* __restrict__ src_rank, int64_t N,
+                                                                 const I* __restrict__ src_rank, int64_t N,
                                                                  int32_t R, const int32_t* __restrict__ num_runs,
                                                                  int32_t* __restrict__ run_offsets,
                                                                  int32_t* __restrict__ rank_runs,
@@ -332,7 +339,7 @@ __global__ __launch_bounds__(kScanBlock) void run_offsets_kernel(const int32_t* 
   if (f) {
     const int32_t run = before + __popcll(m & lt);
     run_offsets[run] = (int32_t)a;
-    const int32_t r = src_rank[a];
+    const int32_t r = (int32_t)src_rank[a];
     if (r >= 0 && r < R) {
       if (lds) atomicAdd(&cnt[r], 1);
       else atomicAdd(&rank_runs[r], 1);
@@ -353,9 +360,9 @@ __global__ __launch_bounds__(kScanBlock) void run_offsets_kernel(const int32_t* 
 // rows.  One wave per run (four to a block): a lane takes four 16-byte chunks
 // of a row at a time and two rows together, so that a wave has up to 8 KB on
 // its way behind one read of the run's positions; rows are added in order.
-template <class E>
+template <class E, class I>
 __global__ __launch_bounds__(256) void run_combine_kernel(const bf16_t* __restrict__ Y,
-                                                          const int32_t* __restrict__ pos,
+                                                          const I* __restrict__ pos,
                                                           const bf16_t* __restrict__ w,
                                                           const int32_t* __restrict__ run_offsets,
                                                           const int32_t* __restrict__ num_runs, int64_t H,
@@ -370,7 +377,7 @@ __global__ __launch_bounds__(256) void run_combine_kernel(const bf16_t* __restri
     float acc[U][8] = {};
     for (int32_t a0 = b; a0 < e; a0 += 64) {
       const int n = e - a0 < 64 ? e - a0 : 64;
-      const int32_t my_pos = lane < n ? pos[a0 + lane] : 0;
+      const int32_t my_pos = lane < n ? (int32_t)pos[a0 + lane] : 0;
       const int32_t my_w = lane < n ? (int32_t)w[a0 + lane] : 0;
       auto load = [&](int j, uint4 (&v)[U]) __attribute__((always_inline)) {
         const uint4* row = reinterpret_cast<const uint4*>(Y + (int64_t)__builtin_amdgcn_readlane(my_pos, j) * H);
@@ -423,11 +430,16 @@ size_t pmx_ep_payload_workspace_bytes(int64_t num_assign, int32_t num_ranks) {
          256;
 }
 
-int pmx_ep_dispatch_payload(const int32_t* phys, const void* hidden, const void* weights, int64_t T, int32_t K,
+}  // extern "C"
+
+namespace {
+
+template <class I>
+int ep_dispatch_payload_t(const I* phys, const void* hidden, const void* weights, int64_t T, int32_t K,
                             int64_t H, int32_t R, int32_t slots_per_rank, int32_t* assign_counts,
                             int32_t* assign_offsets, int32_t* unique_counts, int32_t* unique_offsets,
-                            void* send_hidden, int32_t* unique_tokens, int32_t* send_meta, void* send_weights,
-                            int32_t* target_rank, int32_t* status, void* workspace, size_t workspace_bytes,
+                            void* send_hidden, I* unique_tokens, int32_t* send_meta, void* send_weights,
+                            I* target_rank, int32_t* status, void* workspace, size_t workspace_bytes,
                             pmx_stream_t stream) {
   if (T < 0 || K <= 0 || K > kPayloadMaxTopK || H < 0 || R <= 0 || slots_per_rank <= 0) return PMX_ERR_ARG;
   if (R > kPayloadMaxRanks) return PMX_ERR_ARG;
@@ -463,8 +475,8 @@ int pmx_ep_dispatch_payload(const int32_t* phys, const void* hidden, const void*
   const unsigned chunks = (unsigned)g.nchunks;
   int nbits = 0;
   while ((1 << nbits) < R) ++nbits;
-  auto hist = lds ? payload_hist_kernel<true> : payload_hist_kernel<false>;
-  auto place = lds ? payload_place_kernel<true> : payload_place_kernel<false>;
+  auto hist = lds ? payload_hist_kernel<true, I> : payload_hist_kernel<false, I>;
+  auto place = lds ? payload_place_kernel<true, I> : payload_place_kernel<false, I>;
   hist<<<chunks, 64, lds_bytes, stream>>>(phys, A, K, R, slots_per_rank, g.seg, g.chunk, nbits, target_rank, table, flags,
                                           status);
   PMX_LAUNCH_CHECK();
@@ -484,6 +496,32 @@ int pmx_ep_dispatch_payload(const int32_t* phys, const void* hidden, const void*
   return PMX_OK;
 }
 
+}  // namespace
+
+extern "C" {
+
+int pmx_ep_dispatch_payload(const int32_t* phys, const void* hidden, const void* weights, int64_t T, int32_t K,
+                            int64_t H, int32_t R, int32_t slots_per_rank, int32_t* assign_counts,
+                            int32_t* assign_offsets, int32_t* unique_counts, int32_t* unique_offsets,
+                            void* send_hidden, int32_t* unique_tokens, int32_t* send_meta, void* send_weights,
+                            int32_t* target_rank, int32_t* status, void* workspace, size_t workspace_bytes,
+                            pmx_stream_t stream) {
+  return ep_dispatch_payload_t(phys, hidden, weights, T, K, H, R, slots_per_rank, assign_counts, assign_offsets,
+                               unique_counts, unique_offsets, send_hidden, unique_tokens, send_meta, send_weights,
+                               target_rank, status, workspace, workspace_bytes, stream);
+}
+
+int pmx_ep_dispatch_payload_i64(const int64_t* phys, const void* hidden, const void* weights, int64_t T, int32_t K,
+                            int64_t H, int32_t R, int32_t slots_per_rank, int32_t* assign_counts,
+                            int32_t* assign_offsets, int32_t* unique_counts, int32_t* unique_offsets,
+                            void* send_hidden, int64_t* unique_tokens, int32_t* send_meta, void* send_weights,
+                            int64_t* target_rank, int32_t* status, void* workspace, size_t workspace_bytes,
+                            pmx_stream_t stream) {
+  return ep_dispatch_payload_t(phys, hidden, weights, T, K, H, R, slots_per_rank, assign_counts, assign_offsets,
+                               unique_counts, unique_offsets, send_hidden, unique_tokens, send_meta, send_weights,
+                               target_rank, status, workspace, workspace_bytes, stream);
+}
+
 size_t pmx_ep_combine_workspace_bytes(int64_t num_recv) {
   if (num_recv < 0) return 0;
   const int64_t nblocks = (num_recv + kScanBlock - 1) / kScanBlock + 1;
@@ -494,9 +532,8 @@ size_t pmx_ep_combine_workspace_bytes(int64_t num_recv) {
 
 namespace {
 
-template <class E>
-int ep_combine_aggregate_t(const void* Y, const int32_t* pos, const void* w, const int32_t* src_rank,
-                             const int32_t* src_token, int64_t N, int64_t H, int32_t R, void* out,
+template <class E, class I>
+int ep_combine_aggregate_t(const void* Y, const I* pos, const void* w, const I* src_rank, const I* src_token, int64_t N, int64_t H, int32_t R, void* out,
                              int32_t* run_offsets, int32_t* rank_runs, int32_t* num_runs, int32_t* status,
                              void* workspace, size_t workspace_bytes, pmx_stream_t stream) {
   if (N < 0 || H < 0 || R <= 0) return PMX_ERR_ARG;
@@ -528,7 +565,7 @@ int ep_combine_aggregate_t(const void* Y, const int32_t* pos, const void* w, con
                                                                    run_offsets, rank_runs, status);
   PMX_LAUNCH_CHECK();
   if (H > 0) {
-    run_combine_kernel<E><<<(unsigned)((N + 3) / 4), 256, 0, stream>>>(static_cast<const bf16_t*>(Y), pos,
+    run_combine_kernel<E, I><<<(unsigned)((N + 3) / 4), 256, 0, stream>>>(static_cast<const bf16_t*>(Y), pos,
                                                         static_cast<const bf16_t*>(w), run_offsets, num_runs, H,
                                                         static_cast<bf16_t*>(out));
     PMX_LAUNCH_CHECK();
@@ -545,16 +582,31 @@ int pmx_ep_combine_aggregate(const void* Y, const int32_t* pos, const void* w, c
                              int32_t* run_offsets, int32_t* rank_runs, int32_t* num_runs, int32_t* status,
                              void* workspace, size_t workspace_bytes, pmx_stream_t stream) {
   return ep_combine_aggregate_t<EltBF16>(Y, pos, w, src_rank, src_token, N, H, R, out, run_offsets, rank_runs,
-                                        num_runs, status, workspace, workspace_bytes, stream);
+                                     num_runs, status, workspace, workspace_bytes, stream);
 }
 
 int pmx_ep_combine_aggregate_f16(const void* Y, const int32_t* pos, const void* w, const int32_t* src_rank,
-                                 const int32_t* src_token, int64_t N, int64_t H, int32_t R, void* out,
-                                 int32_t* run_offsets, int32_t* rank_runs, int32_t* num_runs, int32_t* status,
-                                 void* workspace, size_t workspace_bytes, pmx_stream_t stream) {
+                             const int32_t* src_token, int64_t N, int64_t H, int32_t R, void* out,
+                             int32_t* run_offsets, int32_t* rank_runs, int32_t* num_runs, int32_t* status,
+                             void* workspace, size_t workspace_bytes, pmx_stream_t stream) {
   return ep_combine_aggregate_t<EltF16>(Y, pos, w, src_rank, src_token, N, H, R, out, run_offsets, rank_runs,
-                                        num_runs, status, workspace, workspace_bytes, stream);
+                                     num_runs, status, workspace, workspace_bytes, stream);
 }
 
+int pmx_ep_combine_aggregate_i64(const void* Y, const int64_t* pos, const void* w, const int64_t* src_rank,
+                             const int64_t* src_token, int64_t N, int64_t H, int32_t R, void* out,
+                             int32_t* run_offsets, int32_t* rank_runs, int32_t* num_runs, int32_t* status,
+                             void* workspace, size_t workspace_bytes, pmx_stream_t stream) {
+  return ep_combine_aggregate_t<EltBF16>(Y, pos, w, src_rank, src_token, N, H, R, out, run_offsets, rank_runs,
+                                     num_runs, status, workspace, workspace_bytes, stream);
+}
+
+int pmx_ep_combine_aggregate_i64_f16(const void* Y, const int64_t* pos, const void* w, const int64_t* src_rank,
+                             const int64_t* src_token, int64_t N, int64_t H, int32_t R, void* out,
+                             int32_t* run_offsets, int32_t* rank_runs, int32_t* num_runs, int32_t* status,
+                             void* workspace, size_t workspace_bytes, pmx_stream_t stream) {
+  return ep_combine_aggregate_t<EltF16>(Y, pos, w, src_rank, src_token, N, H, R, out, run_offsets, rank_runs,
+                                     num_runs, status, workspace, workspace_bytes, stream);
+}
 
 }  // extern "C"

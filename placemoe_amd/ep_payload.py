@@ -5,7 +5,7 @@ PlaceMoE's dispatch and combine around the all-to-all, on the GPU.
 (veomni/distributed/moe/hiermoe/all_to_all.py:979-1055): it returns the same
 seven values - ``(send_hidden, send_meta, send_weights, unique_tokens,
 unique_send_splits, assignment_send_splits, target_ranks)`` - computed by
-``pmx_ep_dispatch_payload``.  ``aggregate_weighted_outputs`` mirrors
+``pmx_ep_dispatch_payload_i64``.  ``aggregate_weighted_outputs`` mirrors
 ``_aggregate_weighted_outputs`` (:2266-2294) and ``combine_aggregate`` fuses
 it with the unsort and weighting of ``rank_dedup_combine`` (:2553-2556),
 both through ``pmx_ep_combine_aggregate``.  The split lists are host lists,
@@ -54,7 +54,7 @@ def build_local_payload(hidden_states: torch.Tensor, selected_experts: torch.Ten
     T, K = int(routed.shape[0]), int(routed.shape[1])
     H = int(hidden_states.shape[-1])
     A = T * K
-    phys = routed.to(device=device, dtype=torch.int32).contiguous()
+    phys = routed.to(device=device, dtype=torch.int64).contiguous()
     weights = routing_weights.to(device=device, dtype=dt).contiguous()
     hidden = hidden_states.contiguous()
     pad = (-H) % 8
@@ -69,13 +69,13 @@ def build_local_payload(hidden_states: torch.Tensor, selected_experts: torch.Ten
     assign_offsets = torch.empty(ep_size + 1, **i32)
     unique_offsets = torch.empty(ep_size + 1, **i32)
     send_hidden = torch.empty((A, Hp), dtype=dt, device=device)
-    unique_tokens = torch.empty(A, **i32)
+    unique_tokens = torch.empty(A, dtype=torch.int64, device=device)
     send_meta = torch.empty((A, 3), **i32)
     send_weights = torch.empty(A, dtype=dt, device=device)
-    target_rank = torch.empty(A, **i32)
+    target_rank = torch.empty(A, dtype=torch.int64, device=device)
     ws = _workspace(_capi.load().pmx_ep_payload_workspace_bytes(A, ep_size), device)
     _capi.call(
-        "pmx_ep_dispatch_payload", phys.data_ptr() if A else None, hidden.data_ptr() if T else None,
+        "pmx_ep_dispatch_payload_i64", phys.data_ptr() if A else None, hidden.data_ptr() if T else None,
         weights.data_ptr() if A else None, T, K, Hp, ep_size, num_local, assign_counts.data_ptr(),
         assign_offsets.data_ptr(), unique_counts.data_ptr(), unique_offsets.data_ptr(),
         send_hidden.data_ptr() if A else None, unique_tokens.data_ptr() if A else None,
@@ -92,10 +92,10 @@ def build_local_payload(hidden_states: torch.Tensor, selected_experts: torch.Ten
         send_hidden[:U, :H].to(hidden_states.dtype),
         send_meta,
         send_weights.to(routing_weights.dtype).unsqueeze(1),
-        unique_tokens[:U].to(torch.long),
+        unique_tokens[:U],
         unique_send_splits,
         assignment_send_splits,
-        target_rank.reshape(T, K).to(torch.long),
+        target_rank.reshape(T, K),
     )
 
 
@@ -117,18 +117,18 @@ def combine_aggregate(expert_outputs: torch.Tensor, pos: torch.Tensor, recv_weig
         y = torch.nn.functional.pad(y, (0, pad))
     Hp = H + pad
     i32 = dict(dtype=torch.int32, device=device)
-    pos32 = pos.to(**i32).contiguous()
+    index = (pos, source_ranks, source_token_indices)
+    wide = all(t.dtype == torch.int64 for t in index)  # read as they are; other types as int32
+    pos, ranks, tokens = (t.to(device=device, dtype=torch.int64 if wide else torch.int32).contiguous() for t in index)
     w = recv_weights.reshape(-1).to(device=device, dtype=dt).contiguous()
-    ranks = source_ranks.to(**i32).contiguous()
-    tokens = source_token_indices.to(**i32).contiguous()
     out = torch.empty((max(N, 1), Hp), dtype=dt, device=device)
     run_offsets = torch.empty(N + 1, **i32)
     host_counts = torch.zeros(ep_size + 2, **i32)
     rank_runs, num_runs, status = host_counts.split([ep_size, 1, 1])
     ws = _workspace(_capi.load().pmx_ep_combine_workspace_bytes(N), device)
-    name = "pmx_ep_combine_aggregate_f16" if dt == torch.float16 else "pmx_ep_combine_aggregate"
+    name = "pmx_ep_combine_aggregate" + ("_i64" if wide else "") + ("_f16" if dt == torch.float16 else "")
     _capi.call(
-        name, y.data_ptr(), pos32.data_ptr() if N else None, w.data_ptr() if N else None,
+        name, y.data_ptr(), pos.data_ptr() if N else None, w.data_ptr() if N else None,
         ranks.data_ptr() if N else None, tokens.data_ptr() if N else None, N, Hp, ep_size, out.data_ptr(),
         run_offsets.data_ptr(), rank_runs.data_ptr(), num_runs.data_ptr(), status.data_ptr(), ws.data_ptr(),
         ws.numel(), _stream(device),

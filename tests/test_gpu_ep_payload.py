@@ -8,6 +8,7 @@ import pytest
 import torch
 
 from oracle import moe_oracle as O
+from placemoe_amd import _capi
 from placemoe_amd import ep_payload as EP
 from placemoe_amd import kernels
 from placemoe_amd.workloads import make_workload
@@ -148,3 +149,39 @@ def test_combine_aggregate_run_lengths(cuda, H):
     ref, rsplits = O.aggregate_weighted_outputs(weighted, tokens, splits)
     assert gsplits == rsplits
     assert_bf16_close(got.cpu(), ref)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("N,R", [(1, 1), (1000, 3), (5000, 5000)])
+def test_combine_aggregate_of_either_index_type(cuda, N, R, dtype):
+    g = torch.Generator(device=cuda).manual_seed(N)
+    ranks = torch.sort(torch.randint(0, R, (N,), generator=g, device=cuda)).values
+    tokens = torch.arange(N, device=cuda) // 3
+    y = torch.randn((N, 72), generator=g, device=cuda).to(dtype)
+    pos, w = torch.randperm(N, generator=g, device=cuda), torch.rand((N,), generator=g, device=cuda).to(dtype)
+    got, splits = EP.combine_aggregate(y, pos, w, ranks, tokens, R)
+    ref, ref_splits = EP.combine_aggregate(y, pos.int(), w, ranks.int(), tokens.int(), R)
+    mixed, mixed_splits = EP.combine_aggregate(y, pos, w, ranks.int(), tokens, R)
+    assert splits == ref_splits == mixed_splits and torch.equal(got, ref) and torch.equal(got, mixed)
+
+
+def test_payload_of_int32_slots_through_the_c_entry(cuda):
+    T, K, R, L, H = 300, 6, 4, 5, 16
+    g = torch.Generator(device=cuda).manual_seed(2)
+    phys = torch.randint(0, R * L, (T, K), generator=g, device=cuda)
+    hidden = torch.randn((T, H), generator=g, device=cuda).to(torch.bfloat16)
+    w = torch.rand((T, K), generator=g, device=cuda).to(torch.bfloat16)
+    want = EP.build_local_payload(hidden, phys, w, R * L, R)
+    A = T * K
+    i32 = lambda *s: torch.zeros(s, dtype=torch.int32, device=cuda)
+    p32, ac, ao, uc, uo = phys.int(), i32(R), i32(R + 1), i32(R), i32(R + 1)
+    sh, sw = torch.zeros((A, H), dtype=torch.bfloat16, device=cuda), torch.zeros(A, dtype=torch.bfloat16, device=cuda)
+    ut, meta, tr, status = i32(A), i32(A, 3), i32(A), i32(1)
+    ws = torch.empty(_capi.load().pmx_ep_payload_workspace_bytes(A, R), dtype=torch.uint8, device=cuda)
+    _capi.call("pmx_ep_dispatch_payload", *(t.data_ptr() for t in (p32, hidden, w)), T, K, H, R, L,
+               *(t.data_ptr() for t in (ac, ao, uc, uo, sh, ut, meta, sw, tr, status, ws)), ws.numel(),
+               torch.cuda.current_stream(cuda).cuda_stream)
+    U = int(uo[-1])
+    assert uc.tolist() == want[4] and ac.tolist() == want[5] and int(ao[-1]) == A and U == sum(want[4])
+    assert torch.equal(sh[:U], want[0]) and torch.equal(meta, want[1]) and torch.equal(sw[:, None], want[2])
+    assert torch.equal(ut[:U].long(), want[3]) and torch.equal(tr.view(T, K).long(), want[6])
