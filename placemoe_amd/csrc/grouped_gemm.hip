@@ -2255,13 +2255,17 @@ constexpr bool use_w4() { return PMX_GEMM_W4 && ((PMX_W4_KINDS >> KIND) & 1); }
 using Few64 = fr::Cfg<1, 4, 4, 2, 2, 3, 2>;   // 64 x 128 tiles, 24 KB stages
 using Few128 = fr::Cfg<2, 4, 4, 4, 2, 3, 1>;  // 128 x 256 tiles, 48 KB stages
 constexpr int64_t kFewRows64[4] = {40, 48, 40, 40};  // fc1, fc2, fc1 dgrad, fc2 dgrad
-constexpr int64_t kFewRows128[4] = {208, 48, 40, 120};
+// fc1 goes no further than 128 rows: under Zipf(1.0) most rows lie in large
+// copies (101 copies of 1280 x 768, 174 rows on average: 169 / 145 us).
+constexpr int64_t kFewRows128[4] = {128, 48, 40, 120};
 // Weight gradients (us, fc2 + fc1; few-rows / four-wave kernel; 2048 x 768
 // unless stated): 160 copies of 5 rows 90 + 169 / 108 + 195, of 25 rows 85 +
 // 163 / 109 + 203, of 96 rows 102 + 215 / 128 + 240, 128 copies of 128 rows 100
 // + 200 / 113 + 208, of 256 rows 148 + 290 / 146 + 278; 32 copies of 60 rows of
 // 4096 x 1536 75 + 150 / 91 + 170.
-constexpr int64_t kFewRowsWgrad = 128;
+// The average says nothing of the hottest copies, whose K-tiles this kernel
+// loads one at a time: the line lies where even they have few.
+constexpr int64_t kFewRowsWgrad = 48;
 
 template <int KIND, class CF>
 int launch_few(const GemmParams& P, int cus, hipStream_t stream) {
@@ -2278,10 +2282,10 @@ int launch(const GemmParams& P, hipStream_t stream) {
   const int grid = grid_size();
   if (grid <= 0) return PMX_ERR_HIP;
   if constexpr (KIND == KIND_TN) {
-    const int64_t few_tiles = P.G * ((P.M + fr::kWgT - 1) / fr::kWgT) * ((P.N + fr::kWgT - 1) / fr::kWgT);
-    if (PMX_FEW_ROWS && P.K <= kFewRowsWgrad * P.G && few_tiles < (int64_t)1 << 30) {
-      const unsigned blocks = (unsigned)((few_tiles + kNumXcd - 1) / kNumXcd * kNumXcd);
-      fr::few_rows_wgrad_grouped_gemm_kernel<<<blocks, fr::kWgNT, 0, stream>>>(P);
+    const int64_t tiles = ((P.M + fr::kWgT - 1) / fr::kWgT) * ((P.N + fr::kWgT - 1) / fr::kWgT);
+    const int64_t blocks = P.G * ((tiles + kNumXcd - 1) / kNumXcd) * kNumXcd;
+    if (PMX_FEW_ROWS && P.K <= kFewRowsWgrad * P.G && blocks < (int64_t)1 << 30) {
+      fr::few_rows_wgrad_grouped_gemm_kernel<<<(unsigned)blocks, fr::kWgNT, 0, stream>>>(P);
       PMX_LAUNCH_CHECK();
       return PMX_OK;
     }

@@ -127,7 +127,8 @@ def test_fc1_with_row_weights_is_fc1_then_weight_rows(cuda, counts, H, I, dtype)
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
 @pytest.mark.parametrize("split", [False, True])
 @pytest.mark.parametrize("counts,M,N", [([1, 0, 31, 32, 33, 63, 64, 65, 0, 129], 264, 136), ([128], 128, 128),
-                                        ([0, 0, 0, 5], 8, 1024), ([200, 0, 56], 400, 72), ([90] * 20, 136, 200)])
+                                        ([0, 0, 0, 5], 8, 1024), ([200, 0, 56], 400, 72), ([90] * 20, 136, 200),
+                                        ([0, 0, 0, 300, 0, 0, 0], 400, 72), ([3, 190] + [1] * 7, 1160, 1032)])
 def test_weight_gradient(cuda, counts, M, N, split, dtype):
     """Few rows per copy: against fp32 products and the 256-row kernels; empty
     copies are zero, rows past the last copy (NaN here) reach nothing."""
