@@ -2329,9 +2329,9 @@ int launch(const GemmParams& P, hipStream_t stream) {
     // two K-tiles to land, as for fc2 and the fc1 dgrad (us, register-staged /
     // four-wave: 128 copies of 256 rows of 2048 x 768 302 / 325).  Above it the
     // four-wave kernel: at 400-500 rows it takes 1-6% longer by itself (400
-    // rows 414-444 / 404), but its loads draw less power, and the GEMMs that
-    // follow run 2% faster (256 copies of 512 rows, training step with fold:
-    // 6077 us against 6216 with the register-staged fc1).
+    // rows 414-444 / 404), but draws less power, and a training step over 256
+    // copies of 512 rows gained nothing from the other (6216 us against
+    // 6153-6257 without it on three boxes).
     // Row weights (non-EP) too: the four-wave epilogue has no register left for
     // them (2 spill), and a separate pass over act costs more than the 1-3%
     // between the kernels.
