@@ -325,25 +325,17 @@ __global__ __launch_bounds__(CF::NT, CF::NW * CF::BPC / 4) void few_rows_grouped
   // Issue cursor: NST - 1 K-tiles in front of the one being multiplied.
   Tile<KIND, CF> it;
   int64_t i_tile = first;
+  // Every tile walks K from 0 as the 256-row kernels do: an output's bits depend
+  // on its row and its copy's weights alone, not on the slot that holds the copy
+  // or on how many rows the call has.  (Tiles that start at K-tiles of their own
+  // spread the K-contiguous weights' reads over the memory channels, but sum in an
+  // order of the slot; fc1 183 -> 178 us at 160 copies of 5 rows of 2048 x 768,
+  // 158 -> 149 at 32 of 20 rows of 4096 x 1536.)
   int32_t i_kt = 0;
   bool i_live = true;
-  // K-contiguous weights: the rows of a K-tile lie K*2 bytes apart, often a
-  // power of two, so that at one K-tile all blocks read addresses alike in
-  // their low bits and crowd a part of the memory channels.  Each tile
-  // therefore starts at its own K-tile and wraps around (tiles that share a
-  // weight strip start alike): fc1 203 -> 175 us at 160 copies of 5 rows
-  // (2048 x 768), 170 -> 143 us at 32 copies of 20 rows (4096 x 1536).  [K][N]
-  // weights spread by themselves (no change, +-2%).
-  int32_t i_rot = 0;
-  auto next_kt = [&]() {
-    if constexpr (b_is_mn<KIND>()) return i_kt;
-    const int32_t k = i_kt + i_rot;
-    return k >= nk ? k - nk : k;
-  };
   auto set_tile = [&]() {
     decode(i_tile, it.i);
     setup<KIND, CF>(P, it, wave, lane);
-    if constexpr (!b_is_mn<KIND>()) i_rot = (it.i.g * 5 + it.i.ntile * 3) % nk;
   };
   set_tile();
   int i_stage = 0;
@@ -367,7 +359,7 @@ __global__ __launch_bounds__(CF::NT, CF::NW * CF::BPC / 4) void few_rows_grouped
 #pragma unroll
   for (int s = 0; s < CF::NST - 1; ++s) {
     static_for<0, L>([&](auto j) __attribute__((always_inline)) {
-      issue<KIND, CF, decltype(j)::value>(P, lds + i_stage * CF::STAGE, it, next_kt(), wave);
+      issue<KIND, CF, decltype(j)::value>(P, lds + i_stage * CF::STAGE, it, i_kt, wave);
     });
     advance_issue();
   }
@@ -419,7 +411,7 @@ __global__ __launch_bounds__(CF::NT, CF::NW * CF::BPC / 4) void few_rows_grouped
       constexpr int j = decltype(jj)::value;
       if constexpr (decltype(loads)::value) {
         static_for<j * L / NR, (j + 1) * L / NR>([&](auto l) __attribute__((always_inline)) {
-          issue<KIND, CF, decltype(l)::value>(P, refill, it, next_kt(), wave);
+          issue<KIND, CF, decltype(l)::value>(P, refill, it, i_kt, wave);
         });
       }
       read(Int<order<CF>(j)>{}, stage, ks, fr);

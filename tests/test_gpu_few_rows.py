@@ -150,3 +150,35 @@ def test_weight_gradient(cuda, counts, M, N, split, dtype):
         s = int(off[g])
         want = a[s:s + n].float().t() @ b[s:s + n].float() if n else torch.zeros((M, N), device=cuda)
         assert_bf16_close(got[g], want, name=f"copy {g} ({n} rows)")
+
+
+def _all_kinds(x, dy, w1, w2, counts):
+    off = _off(counts)
+    G, I = len(counts), w2.shape[2]
+    offd = torch.as_tensor(off, dtype=torch.int32, device=x.device)
+    up = w1.view(-1)[I * x.shape[1]:]
+    gu, act = kernels.gemm_fc1_swiglu(x, w1, up, 2 * I * x.shape[1], offd, G, I)
+    dg1 = kernels.gemm_fc2_dgrad_swiglu(dy, w2, gu, offd)
+    return {"gu": gu, "act": act, "y": kernels.group_gemm_nt(act, w2, offd), "dg1": dg1,
+            "dx": kernels.group_gemm_nn(dg1, w1, offd)}
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
+def test_bits_depend_on_neither_the_copy_nor_the_batch(cuda, dtype):
+    """Replicas of one expert give a row the same bits whichever slot serves
+    it, and so do calls with few and with many rows per copy: the placement and
+    the batch a token comes in are not to be seen in its result."""
+    G, H, I, n = 23, 1024, 384, 20
+    gen = torch.Generator(device=cuda).manual_seed(12)
+    rn = lambda *s: torch.randn(s, generator=gen, device=cuda).to(dtype)
+    w1, w2 = (rn(1, 2 * I, H) * 0.03).repeat(G, 1, 1), (rn(1, H, I) * 0.05).repeat(G, 1, 1)
+    x0, dy0 = rn(n, H), rn(n, H)
+    want = {}
+    for extra in (0, 30, 80, 300, 700):  # 20 .. 720 rows per copy: every kernel the kinds run on
+        print(f"few rows, same bits: {dtype} {n + extra} rows per copy", flush=True)
+        x = torch.cat([t for _ in range(G) for t in (x0, rn(extra, H))])
+        dy = torch.cat([t for _ in range(G) for t in (dy0, rn(extra, H))])
+        for k, t in _all_kinds(x, dy, w1, w2, [n + extra] * G).items():
+            t = t.view(G, n + extra, -1)[:, :n]
+            assert torch.equal(t, t[:1].expand_as(t)), f"{k}, {n + extra} rows: the slot changes the bits"
+            assert torch.equal(t[0], want.setdefault(k, t[0].clone())), f"{k}: {n + extra} rows per copy change the bits"
