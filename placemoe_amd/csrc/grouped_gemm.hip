@@ -37,6 +37,7 @@
 //     ds_read_b64_tr_b16, which transpose 4x16 blocks on the way out of LDS.
 
 #include "common.h"
+#include "few_rows_rule.h"
 #include "ktile.h"
 
 // Element type of this build of the file: bf16, or fp16 with -DPMX_ELT_F16
@@ -2228,36 +2229,13 @@ constexpr int64_t kRsMaxRowsPerCopy = 8 * kBM;
 template <int KIND>
 constexpr bool use_w4() { return PMX_GEMM_W4 && ((PMX_W4_KINDS >> KIND) & 1); }
 
-// Copies with few rows (few_rows.h).  The host knows the average rows per copy,
-// M / G, not the counts; two tilings:
-//   64 x 128, two blocks per CU: fc1 and fc2 up to kFewRows64 rows, and the
-//     dgrads where 256-wide tiles would be fewer than the CUs (at most
-//     min(G, M) copies have rows);
-//   128 x 256, one block: up to kFewRows128 rows (the dgrads' [K][N] weights
-//     prefer its 512-byte row segments).
-// Beyond that the kernels above, whose 256-row tiles read each weight strip
-// for twice the rows.  Where the lines lie (us; 64 x 128 / 128 x 256 / 256-row
-// kernels; 2048 x 768 layer, row counts log-normal with sigma 0.5):
-//   copies rows  fc1             fc2             fc2 dgrad       fc1 dgrad
-//   160    4.8   180 / 175 / 265  90 /  91 / 104  95 /  94 / 147 185 / 172 / 193
-//   160    25    185 / 185 / 269 103 / 108 / 107 110 / 108 / 146 207 / 196 / 204
-//   128    96    213 / 195 / 263 119 / 118 / 120 131 / 119 / 141 219 / 198 / 204
-//   128    150   263 / 222 / 270 152 / 129 / 115 167 / 160 / 152 263 / 216 / 210
-//   128    256   391 / 304 / 328 221 / 179 / 148 246 / 207 / 221 383 / 288 / 267
-// and for 16 copies of 7168 x 2048, 12 rows: 159 / 159 / 218, 86 / 83 / 116,
-// 84 / 110 / 184 (a narrow one), 178 / 164 / 193.  fc1 and the fc2 dgrad gain
-// the most: their 256-row kernel's loads have one K-tile to land, those of
-// the register-staged one, which runs fc2 and the fc1 dgrad, two.
+// Copies with few rows (few_rows.h) by the rule of few_rows_rule.h.
 // PMX_FEW_ROWS=0 builds without it (the eight-wave test variant).
 #ifndef PMX_FEW_ROWS
 #define PMX_FEW_ROWS 1
 #endif
 using Few64 = fr::Cfg<1, 4, 4, 2, 2, 3, 2>;   // 64 x 128 tiles, 24 KB stages
 using Few128 = fr::Cfg<2, 4, 4, 4, 2, 3, 1>;  // 128 x 256 tiles, 48 KB stages
-constexpr int64_t kFewRows64[4] = {40, 48, 40, 40};  // fc1, fc2, fc1 dgrad, fc2 dgrad
-// fc1 goes no further than 128 rows: under Zipf(1.0) most rows lie in large
-// copies (101 copies of 1280 x 768, 174 rows on average: 169 / 145 us).
-constexpr int64_t kFewRows128[4] = {128, 48, 40, 120};
 // Weight gradients (us, fc2 + fc1; few-rows / four-wave kernel; 2048 x 768
 // unless stated): 160 copies of 5 rows 90 + 169 / 108 + 195, of 25 rows 85 +
 // 163 / 109 + 203, of 96 rows 102 + 215 / 128 + 240, 128 copies of 128 rows 100
@@ -2315,10 +2293,11 @@ int launch(const GemmParams& P, hipStream_t stream) {
   } else {
     // Weights in two tensors: the few-rows kernel picks one per K-tile.
     const bool few = PMX_FEW_ROWS && P.G <= fr::kMaxG && (KIND != KIND_NN || P.b.split >= P.K || P.b.split % BK == 0);
-    const int64_t copies = P.M < P.G ? P.M : P.G;
-    const bool narrow = KIND == KIND_FC1 || KIND == KIND_NT || copies * ((P.N + BN - 1) / BN) < grid;
-    if (few && narrow && P.M <= kFewRows64[KIND] * P.G) return launch_few<KIND, Few64>(P, grid, stream);
-    if (few && P.M <= kFewRows128[KIND] * P.G) return launch_few<KIND, Few128>(P, grid, stream);
+    const int tiling = few ? pmx::few_rows_tiling(KIND, P.M, P.G, P.N, P.K, grid) : 0;
+    if (tiling == Few64::BM) return launch_few<KIND, Few64>(P, grid, stream);
+    if constexpr (pmx::kFewRowsLines[KIND].max128 > 0) {
+      if (tiling == Few128::BM) return launch_few<KIND, Few128>(P, grid, stream);
+    }
     // FAST: K a multiple of 64, dgrad weights not split (P.b.split >= K).
     // RS (register-staged operands): fc1 and fc2 always; the fc1 dgrad when
     // the copies are small (under 8 m-tiles of rows on average), where each
