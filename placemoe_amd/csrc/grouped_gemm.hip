@@ -2304,18 +2304,16 @@ int launch(const GemmParams& P, hipStream_t stream) {
     // weight strip serves few tiles and its loads wait on memory - with a
     // few large copies the DMA path is faster (it spends less power).
     const bool fast = P.K % BK == 0 && (KIND != KIND_NN || P.b.split >= P.K);
-    // fc1 with up to kRsFc1Rows rows per copy: the register-staged loads, with
-    // two K-tiles to land, as for fc2 and the fc1 dgrad (us, register-staged /
-    // four-wave: 128 copies of 256 rows of 2048 x 768 302 / 325).  Above it the
-    // four-wave kernel: at 400-500 rows it takes 1-6% longer by itself (400
-    // rows 414-444 / 404), but draws less power, and a training step over 256
-    // copies of 512 rows gained nothing from the other (6216 us against
-    // 6153-6257 without it on three boxes).
-    // Row weights (non-EP) too: the four-wave epilogue has no register left for
-    // them (2 spill), and a separate pass over act costs more than the 1-3%
-    // between the kernels.
-    constexpr int64_t kRsFc1Rows = 320;
-    [[maybe_unused]] const bool rs_fc1 = KIND == KIND_FC1 && (P.row_w != nullptr || P.M <= kRsFc1Rows * P.G);
+    // fc1 with row weights (non-EP): the register-staged kernel.  The four-wave
+    // epilogue has no register left for them (2 spill), and a separate pass
+    // over act costs more than there is between the kernels, small layers aside
+    // (with the weights, register-staged / four-wave and pass: 128 copies of 320
+    // rows of 2048 x 768 341 / 394 us, of 2000 rows 1549 / 1585; 32 of 200 rows
+    // 84 / 77, where the launch that falls away makes up for it).  Without row weights the four-wave kernel: the other is
+    // 3-6% faster where copies of 130-320 rows leave their tiles part empty, but
+    // 5-20% slower where they fill them or K is short (40 copies of 240 rows of
+    // 2048 x 1416, even: 211 / 197 us; 12 of 200 rows of 1024 x 2816: 81 / 71).
+    [[maybe_unused]] const bool rs_fc1 = KIND == KIND_FC1 && P.row_w != nullptr;
     if constexpr (use_w4<KIND>()) {
       if (fast && !rs_fc1) {
         w4::grouped_gemm_w4_kernel<KIND><<<grid, w4::NT, 0, stream>>>(P);
