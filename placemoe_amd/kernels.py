@@ -211,6 +211,8 @@ class RouteCheck:
     a graph reports nothing (every replay would write to the word)."""
 
     def __init__(self) -> None:
+        # held by the check: at interpreter exit the module's globals go first
+        self._words = _STATUS_WORDS
         self._word: int | None = None
         self._device: torch.device | None = None
         self._stream = 0
@@ -223,18 +225,18 @@ class RouteCheck:
             self._status, self.checked = 0, True
             return None
         self._device, self._stream = device, stream
-        self._word, address = _STATUS_WORDS.lease()
+        self._word, address = self._words.lease()
         return address
 
     def refused(self) -> None:
         """The launch was refused before anything ran."""
         if self._word is not None:
-            _STATUS_WORDS.give_back(self._word)
+            self._words.give_back(self._word)
             self._word = None
 
     def ready(self) -> bool:
         if self._status is None:
-            _STATUS_WORDS.take(self)
+            self._words.take(self)
         return self._status is not None
 
     def failed(self) -> bool:
@@ -248,7 +250,7 @@ class RouteCheck:
 
     def __del__(self) -> None:
         if self._word is not None:
-            _STATUS_WORDS.orphan(self._word)
+            self._words.orphan(self._word)
 
     def raise_if_failed(self) -> None:
         self.checked = True

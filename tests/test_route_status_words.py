@@ -2,9 +2,14 @@
 in flight gives it up without waiting for the pool's lock."""
 
 import ctypes
+import subprocess
+import sys
 import threading
+from pathlib import Path
 
 from placemoe_amd import kernels
+
+ROOT = Path(__file__).resolve().parents[1]
 
 
 def _pool():
@@ -34,3 +39,16 @@ def test_orphans_come_back_once_written():
     view[b] = 0  # its kernel has run, a's has not
     assert words.lease()[0] == b and list(words._orphans) == [a]
     assert view[b] == words.PENDING
+
+
+def test_checks_pending_at_interpreter_exit_end_quietly():
+    """A serving process ends with its last forward's check unread."""
+    code = """
+from placemoe_amd import experts, kernels
+for word in range(3):
+    check = kernels.RouteCheck()
+    check._word = word  # in flight
+    experts._PENDING_CHECKS.append(check)
+"""
+    out = subprocess.run([sys.executable, "-c", code], cwd=ROOT, capture_output=True, text=True)
+    assert out.returncode == 0 and "Exception ignored" not in out.stderr, out.stderr
