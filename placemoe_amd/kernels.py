@@ -10,6 +10,7 @@ from __future__ import annotations
 
 import ctypes
 import threading
+import time
 from collections import deque
 from dataclasses import dataclass
 
@@ -116,7 +117,7 @@ def route(
     counts = torch.empty(C, dtype=torch.int32, device=dev)
     offsets = torch.empty(C + 1, dtype=torch.int32, device=dev)
     stream = _stream(dev)
-    status_host = check.arm(dev, stream) if check is not None else None
+    status_host = check.arm(dev) if check is not None else None
     try:
         _capi.call(
             "pmx_route_reported", _ptr(sel), _ptr(mapping), _ptr(sources), int(source), S, E, T, K, C,
@@ -215,16 +216,15 @@ class RouteCheck:
         self._words = _STATUS_WORDS
         self._word: int | None = None
         self._device: torch.device | None = None
-        self._stream = 0
         self._status: int | None = None
         self.checked = False
 
-    def arm(self, device: torch.device, stream: int) -> int | None:
-        """The host word's address for a launch on ``stream``."""
+    def arm(self, device: torch.device) -> int | None:
+        """The host word's address for a launch on the device's current stream."""
         if torch.cuda.is_current_stream_capturing():
             self._status, self.checked = 0, True
             return None
-        self._device, self._stream = device, stream
+        self._device = device
         self._word, address = self._words.lease()
         return address
 
@@ -240,12 +240,14 @@ class RouteCheck:
         return self._status is not None
 
     def failed(self) -> bool:
-        if not self.ready():
-            stream = (torch.cuda.ExternalStream(self._stream, device=self._device) if self._stream
-                      else torch.cuda.default_stream(self._device))
-            stream.synchronize()
-            if not self.ready():
-                raise RuntimeError("the routing kernel has run without reporting its status")
+        # Waits for the word itself: the stream's handle may be dead by now, and
+        # other work on the stream or the device need not be waited for.
+        looked = time.monotonic()
+        while not self.ready():
+            time.sleep(20e-6)
+            if time.monotonic() - looked > 1 and not torch.cuda.is_current_stream_capturing():
+                looked = time.monotonic()
+                torch.cuda.current_stream(self._device).query()  # raises if the device's work has ended in an error
         return self._status != 0
 
     def __del__(self) -> None:

@@ -7,6 +7,9 @@ import sys
 import threading
 from pathlib import Path
 
+import pytest
+import torch
+
 from placemoe_amd import kernels
 
 ROOT = Path(__file__).resolve().parents[1]
@@ -52,3 +55,38 @@ for word in range(3):
 """
     out = subprocess.run([sys.executable, "-c", code], cwd=ROOT, capture_output=True, text=True)
     assert out.returncode == 0 and "Exception ignored" not in out.stderr, out.stderr
+
+
+def test_waiting_uses_no_stream(monkeypatch):
+    """A wait ends when the word lands; the stream of the launch, which its
+    owner may have destroyed since, is not touched."""
+    words, view = _pool()
+    monkeypatch.setattr(kernels, "_STATUS_WORDS", words)
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    for name in ("ExternalStream", "default_stream", "synchronize"):
+        monkeypatch.setattr(torch.cuda, name, lambda *a, **k: pytest.fail("waits on a stream or the device"))
+    for status in (0, 1):
+        check = kernels.RouteCheck()
+        check._word, _ = words.lease()
+        check._device = torch.device("cuda", 0)
+        kernel = threading.Timer(0.1, view.__setitem__, (check._word, status))
+        kernel.start()
+        assert check.failed() == bool(status)
+        kernel.join()
+    assert sorted(words._free) == [0, 1, 2]
+
+
+def test_waiting_raises_what_ended_the_device(monkeypatch):
+    words, _ = _pool()
+    monkeypatch.setattr(kernels, "_STATUS_WORDS", words)
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+
+    class Dead:
+        def query(self):
+            raise RuntimeError("device error")
+
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda device: Dead())
+    check = kernels.RouteCheck()
+    check._word, _ = words.lease()
+    with pytest.raises(RuntimeError, match="device error"):
+        check.failed()
