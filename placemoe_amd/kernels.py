@@ -205,6 +205,14 @@ class _StatusWords:
 _STATUS_WORDS = _StatusWords()
 
 
+def _capturing(device: torch.device) -> bool:
+    """Whether the device's current stream is being captured."""
+    if device.index == torch.cuda.current_device():
+        return torch.cuda.is_current_stream_capturing()
+    with torch.cuda.device(device):
+        return torch.cuda.is_current_stream_capturing()
+
+
 class RouteCheck:
     """The routing status word of one ``route`` call, stored to pinned host
     memory by the routing kernel itself.  ``ready()`` asks (without waiting)
@@ -221,7 +229,7 @@ class RouteCheck:
 
     def arm(self, device: torch.device) -> int | None:
         """The host word's address for a launch on the device's current stream."""
-        if torch.cuda.is_current_stream_capturing():
+        if _capturing(device):
             self._status, self.checked = 0, True
             return None
         self._device = device
@@ -245,7 +253,7 @@ class RouteCheck:
         looked = time.monotonic()
         while not self.ready():
             time.sleep(20e-6)
-            if time.monotonic() - looked > 1 and not torch.cuda.is_current_stream_capturing():
+            if time.monotonic() - looked > 1 and not _capturing(self._device):
                 looked = time.monotonic()
                 torch.cuda.current_stream(self._device).query()  # raises if the device's work has ended in an error
         return self._status != 0

@@ -1,6 +1,7 @@
 """Host side of the routing status words: a check that ends while its word is
 in flight gives it up without waiting for the pool's lock."""
 
+import contextlib
 import ctypes
 import subprocess
 import sys
@@ -21,6 +22,22 @@ def _pool():
     words._blocks.append((None, ctypes.addressof(view), view))
     words._free = [0, 1, 2]
     return words, view
+
+
+def _devices(monkeypatch, capturing):
+    """torch.cuda of a host whose device 0 is current; the streams of the
+    devices in ``capturing`` are being captured."""
+    current = [0]
+
+    @contextlib.contextmanager
+    def device(d):
+        current.append(torch.device(d).index)
+        yield
+        current.pop()
+
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: current[-1])
+    monkeypatch.setattr(torch.cuda, "device", device)
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: current[-1] in capturing)
 
 
 def test_a_check_that_ends_does_not_wait_for_the_lock():
@@ -62,7 +79,7 @@ def test_waiting_uses_no_stream(monkeypatch):
     owner may have destroyed since, is not touched."""
     words, view = _pool()
     monkeypatch.setattr(kernels, "_STATUS_WORDS", words)
-    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    _devices(monkeypatch, capturing=())
     for name in ("ExternalStream", "default_stream", "synchronize"):
         monkeypatch.setattr(torch.cuda, name, lambda *a, **k: pytest.fail("waits on a stream or the device"))
     for status in (0, 1):
@@ -79,7 +96,7 @@ def test_waiting_uses_no_stream(monkeypatch):
 def test_waiting_raises_what_ended_the_device(monkeypatch):
     words, _ = _pool()
     monkeypatch.setattr(kernels, "_STATUS_WORDS", words)
-    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    _devices(monkeypatch, capturing=())
 
     class Dead:
         def query(self):
@@ -88,5 +105,20 @@ def test_waiting_raises_what_ended_the_device(monkeypatch):
     monkeypatch.setattr(torch.cuda, "current_stream", lambda device: Dead())
     check = kernels.RouteCheck()
     check._word, _ = words.lease()
+    check._device = torch.device("cuda", 0)
     with pytest.raises(RuntimeError, match="device error"):
         check.failed()
+
+
+@pytest.mark.parametrize("capturing", [0, 1])
+@pytest.mark.parametrize("launch", [0, 1])
+def test_capture_is_asked_of_the_launch_device(monkeypatch, launch, capturing):
+    """A routing captured on its own device leases no word (every replay would
+    write to it); one beside another device's capture does."""
+    words, _ = _pool()
+    monkeypatch.setattr(kernels, "_STATUS_WORDS", words)
+    _devices(monkeypatch, capturing=(capturing,))
+    check = kernels.RouteCheck()
+    address = check.arm(torch.device("cuda", launch))
+    assert (address is None) == check.checked == (launch == capturing)
+    assert len(words._free) == (3 if launch == capturing else 2)
