@@ -127,6 +127,10 @@ def route(
         if check is not None:
             check.refused()
         raise
+    except _capi.PmxError:  # a launch failed, others of the call may run
+        if check is not None:
+            check.launch_failed()
+        raise
     return Routing(phys=phys, counts=counts, offsets=offsets, pos=pos, workspace=ws)
 
 
@@ -241,6 +245,19 @@ class RouteCheck:
         if self._word is not None:
             self._words.give_back(self._word)
             self._word = None
+
+    def launch_failed(self) -> None:
+        """A launch of the call failed: what was launched may still write the
+        word, so it is given back only behind the device's work (and stays
+        leased if that cannot be waited for)."""
+        if self._word is None:
+            return
+        try:
+            torch.cuda.synchronize(self._device)
+        except RuntimeError:
+            return
+        if not self.ready():
+            self.refused()
 
     def ready(self) -> bool:
         if self._status is None:

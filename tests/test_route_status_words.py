@@ -11,7 +11,7 @@ from pathlib import Path
 import pytest
 import torch
 
-from placemoe_amd import kernels
+from placemoe_amd import _capi, kernels
 
 ROOT = Path(__file__).resolve().parents[1]
 
@@ -122,3 +122,34 @@ def test_capture_is_asked_of_the_launch_device(monkeypatch, launch, capturing):
     address = check.arm(torch.device("cuda", launch))
     assert (address is None) == check.checked == (launch == capturing)
     assert len(words._free) == (3 if launch == capturing else 2)
+
+
+@pytest.mark.parametrize("written,settles", [(False, True), (True, True), (False, False)])
+def test_a_failed_launch_gives_its_word_back(monkeypatch, written, settles):
+    """The scan may have been launched before the launch that failed: the word
+    comes back once the device has settled, and not before."""
+    words, view = _pool()
+    monkeypatch.setattr(kernels, "_STATUS_WORDS", words)
+    _devices(monkeypatch, capturing=())
+    monkeypatch.setattr(kernels, "_check_dev", lambda *t: torch.device("cpu"))
+    monkeypatch.setattr(kernels, "_stream", lambda device: 0)
+    leased = []
+
+    def fails(name, *args):
+        leased.extend(set(range(3)) - set(words._free))
+        raise _capi.PmxError(name, _capi.PMX_ERR_HIP)
+
+    def synchronize(device):
+        if not settles:
+            raise RuntimeError("device error")
+        if written:
+            view[leased[0]] = 0
+
+    monkeypatch.setattr(_capi, "call", fails)
+    monkeypatch.setattr(torch.cuda, "synchronize", synchronize)
+    check = kernels.RouteCheck()
+    with pytest.raises(_capi.PmxError):
+        kernels.route(torch.zeros((4, 2), dtype=torch.int64), 3, check=check)
+    assert len(leased) == 1
+    assert sorted(words._free) == ([0, 1, 2] if settles else sorted({0, 1, 2} - set(leased)))
+    assert (check._word is None) == settles
