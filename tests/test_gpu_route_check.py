@@ -14,7 +14,7 @@ from placemoe_amd import kernels
 pytestmark = pytest.mark.gpu
 
 
-def _free_words():
+def _words_out():
     w = kernels._STATUS_WORDS
     with w._lock:
         w._collect_orphans()
@@ -39,12 +39,27 @@ def test_status_lands_without_a_synchronisation(cuda, T, K, C, bad):
     assert check.failed() == bad
 
 
+def _spin(seconds):
+    """Keep the current stream busy; the event that follows."""
+    a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+    cycles = 10_000_000
+    torch.cuda._sleep(cycles)
+    a.record()
+    torch.cuda._sleep(cycles)
+    b.record()
+    torch.cuda.synchronize()
+    torch.cuda._sleep(int(cycles * seconds * 1e3 / a.elapsed_time(b)))
+    done = torch.cuda.Event()
+    done.record()
+    return done
+
+
 def test_words_in_flight_are_not_reused(cuda):
     sel = torch.randint(0, 4, (16, 2), device=cuda)
     torch.cuda.synchronize()
     gc.collect()
-    before = _free_words()
-    torch.cuda._sleep(200_000_000)
+    before = _words_out()
+    spin = _spin(2.0)
     held = [kernels.RouteCheck() for _ in range(50)]
     for c in held:
         kernels.route(sel, 4, check=c)
@@ -53,23 +68,24 @@ def test_words_in_flight_are_not_reused(cuda):
     dropped = held[:20]
     del held[:20], dropped, c
     gc.collect()
-    assert _free_words() >= before + 30  # still leased while the kernels wait
+    out = _words_out()  # 30 held, 20 whose checks are gone while their kernels wait
     more = [kernels.RouteCheck() for _ in range(10)]
     for m in more:
         kernels.route(sel, 4, check=m)
-    if not any(h.ready() for h in held):  # the spin still runs
-        assert not words & {m._word for m in more}
+    again = words & {m._word for m in more}
+    assert not spin.query(), "the spin ended before the words were counted"
+    assert out == before + 50 and not again
     torch.cuda.synchronize()
     assert all(c.ready() and not c.failed() for c in held + more)
-    assert _free_words() == before
+    assert _words_out() == before
 
 
 def test_refused_arguments_give_the_word_back(cuda):
-    before = _free_words()
+    before = _words_out()
     check = kernels.RouteCheck()
     with pytest.raises(ValueError):
         kernels.route(torch.zeros((4, 2), dtype=torch.int64, device=cuda), 1 << 25, check=check)
-    assert _free_words() == before
+    assert _words_out() == before
 
 
 def test_captured_routing_replays(cuda):
