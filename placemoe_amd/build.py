@@ -68,8 +68,9 @@ EXTRA_OBJECTS = {"grouped_gemm.f16": ("grouped_gemm.hip", ["-DPMX_ELT_F16"])}
 # name -> (source, extra flags): library variants for tests and comparisons.
 #   tiletab2: a two-entry LDS tile table (the on-the-spot tile decode runs at small shapes);
 #   w8:       the eight-wave GEMM kernel for every call (the four-wave kernel switched off).
-#             It builds without the few-rows kernel too, so that small shapes reach the 256-row kernels.
-VARIANTS = {"tiletab2": ("grouped_gemm.hip", ["-DPMX_TILE_TAB=2"]),
+# Both build without the few-rows kernels, which have no tile table, so that every call reaches
+# the 256-row kernels.
+VARIANTS = {"tiletab2": ("grouped_gemm.hip", ["-DPMX_TILE_TAB=2", "-DPMX_FEW_ROWS=0"]),
             "w8": ("grouped_gemm.hip", ["-DPMX_GEMM_W4=0", "-DPMX_FEW_ROWS=0"])}
 VARIANT_DIR = LIB_DIR / "variants"
 

@@ -2230,7 +2230,7 @@ template <int KIND>
 constexpr bool use_w4() { return PMX_GEMM_W4 && ((PMX_W4_KINDS >> KIND) & 1); }
 
 // Copies with few rows (few_rows.h) by the rule of few_rows_rule.h.
-// PMX_FEW_ROWS=0 builds without it (the eight-wave test variant).
+// PMX_FEW_ROWS=0 builds without it (the test variants).
 #ifndef PMX_FEW_ROWS
 #define PMX_FEW_ROWS 1
 #endif

@@ -4,11 +4,14 @@ calls that measured slower on them than on the 256-row kernels stay off, calls
 that gain stay on, and no call goes past the lines."""
 
 import itertools
+import re
 import shutil
 import subprocess
 from pathlib import Path
 
 import pytest
+
+from tests import test_gpu_few_rows, test_gpu_gemm_bounds
 
 ROOT = Path(__file__).resolve().parents[1]
 KINDS = ("fc1", "fc2", "fc1_dgrad", "fc2_dgrad")
@@ -88,3 +91,27 @@ def test_no_call_goes_past_the_lines(tiling):
         assert bm != 128 or rows <= most128[kind] * g
         if rows <= 8 * g:  # one tile a copy on any kernel: always
             assert bm != 0, (kind, rows, g, H, I)
+
+
+def _wgrad_line():
+    src = (ROOT / "placemoe_amd" / "csrc" / "grouped_gemm.hip").read_text()
+    return int(re.search(r"constexpr int64_t kFewRowsWgrad = (\d+);", src).group(1))
+
+
+def test_gpu_cases_reach_every_few_rows_kernel(tiling):
+    cases = [(int(sum(c)), len(c), H, I) for c, H, I in test_gpu_few_rows.CASES.values() if len(c) <= 1024]
+    reached = {kind: set(tiling([(kind, *c) for c in cases])) for kind in KINDS}
+    assert reached == {"fc1": {0, 64, 128}, "fc2": {0, 64}, "fc1_dgrad": {0, 64, 128}, "fc2_dgrad": {0, 64, 128}}
+    line = _wgrad_line()
+    assert all(sum(c) <= line * len(c) for c, _, _ in test_gpu_few_rows.WGRAD_CASES)
+    assert all(sum(c) > line * len(c) for c, _, _ in test_gpu_few_rows.WGRAD_PAST_THE_LINE)
+
+
+def test_gpu_cases_of_the_256_row_kernels_stay_on_them(tiling):
+    for seed, cases in ((0, test_gpu_gemm_bounds.TILE_TABLE_CASES), (7, test_gpu_gemm_bounds.EIGHT_WAVE_CASES)):
+        for G, A, H, I in cases:
+            rows = int(test_gpu_gemm_bounds._copies(G, A, seed=G + seed)[-1])
+            assert tiling([(kind, rows, G, H, I) for kind in KINDS]) == [0] * 4, (G, A)
+            assert rows > _wgrad_line() * G, (G, A)
+    assert max(G for G, *_ in test_gpu_gemm_bounds.TILE_TABLE_CASES) > 512  # the plain weight-gradient order
+    assert max(G for G, *_ in test_gpu_gemm_bounds.EIGHT_WAVE_CASES) > 512

@@ -6,7 +6,7 @@ rest; the build ``libplacemoe_amd_w8.so`` keeps the 256-row kernels for every
 call.  Both must agree within the bf16 bar over every form the rule accepts:
 copies that end on and next to the tile edges (64, 128), empty copies, one
 copy, as many as the kernel takes (1024) and one more (which goes to the other
-kernels), K off the 64-deep K-tile, columns off the 256-wide tile, split fc1
+kernels), averages past the kernels' lines, K off the 64-deep K-tile, columns off the 256-wide tile, split fc1
 weights whose split is (and is not) a whole number of K-tiles, and top-1 row
 maps with targets outside the output.
 """
@@ -43,6 +43,8 @@ CASES = {
     "edges": (EDGES, 576, 264),
     "edges128": ([128, 127, 129, 60, 200, 100], 320, 136),
     "edges128_tile": ([128, 127, 129, 60, 200, 100], 320, 192),
+    "edges128_below": ([128, 127, 129, 60, 100, 90], 320, 136),
+    "edges128_k_tail": ([128, 127, 129, 60, 100, 90], 200, 264),
     "edges32": ([129, 1, 0, 64, 2, 3, 17, 40], 576, 192),
     "wide": ([1 + i % 29 for i in range(80)] + [0, 63, 64, 65, 128], 1096, 776),
     "k_tail": (EDGES, 200, 72),
@@ -124,11 +126,15 @@ def test_fc1_with_row_weights_is_fc1_then_weight_rows(cuda, counts, H, I, dtype)
         assert torch.equal(got, want)
 
 
+WGRAD_CASES = [([1, 0, 31, 32, 33, 63, 64, 65, 0, 129], 264, 136), ([0, 0, 0, 5], 8, 1024),
+               ([0, 0, 0, 300, 0, 0, 0], 400, 72), ([3, 190] + [1] * 7, 1160, 1032), ([128, 0, 0], 128, 128),
+               ([200, 0, 56, 0, 0, 0], 400, 72), ([90, 0] * 10, 136, 200), ([48], 128, 256)]
+WGRAD_PAST_THE_LINE = [([128], 128, 128), ([200, 0, 56], 400, 72), ([90] * 20, 136, 200)]  # the 256-row kernels
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
 @pytest.mark.parametrize("split", [False, True])
-@pytest.mark.parametrize("counts,M,N", [([1, 0, 31, 32, 33, 63, 64, 65, 0, 129], 264, 136), ([128], 128, 128),
-                                        ([0, 0, 0, 5], 8, 1024), ([200, 0, 56], 400, 72), ([90] * 20, 136, 200),
-                                        ([0, 0, 0, 300, 0, 0, 0], 400, 72), ([3, 190] + [1] * 7, 1160, 1032)])
+@pytest.mark.parametrize("counts,M,N", WGRAD_CASES + WGRAD_PAST_THE_LINE)
 def test_weight_gradient(cuda, counts, M, N, split, dtype):
     """Few rows per copy: against fp32 products and the 256-row kernels; empty
     copies are zero, rows past the last copy (NaN here) reach nothing."""

@@ -10,15 +10,18 @@
 * A block's tiles past its LDS tile table are decoded on the spot.  The test
   build ``libplacemoe_amd_tiletab2.so`` keeps only two table entries, so that
   path runs at small shapes, for every kind and both weight-gradient orders
-  (balanced for G <= 512 copies, plain beyond); its outputs must equal the
-  shipped library's bit for bit (every tile is computed the same way wherever
-  it is decoded) and the fp32 products within the bf16 bar.
+  (balanced for G <= 512 copies, plain beyond; 256 on the four-wave kernel);
+  its outputs must equal the shipped library's bit for bit (every tile is
+  computed the same way wherever it is decoded) and the fp32 products within
+  the bf16 bar.  The cases hold more rows per copy than the few-rows kernels
+  take, which have no tile table (tests/test_few_rows_rule.py checks that on
+  the host).
 * The shipped library runs fc1 + SwiGLU, the fc2 dgrad and the weight
   gradients on the four-wave kernel whenever K is a multiple of 64.  The test
   build ``libplacemoe_amd_w8.so`` runs the eight-wave kernel for every call,
   so its fast-load paths of those kinds stay covered: every kind against the
   fp32 products, and the two builds within the bf16 bar of each other (their
-  MFMA shapes sum in different orders, so the bits may differ).
+  MFMA shapes take 16 and 32 values of K at a time).
 """
 
 import numpy as np
@@ -87,8 +90,10 @@ def _copies(G, A, seed, empty=0.2):
     return off
 
 
-@pytest.mark.parametrize("G,A,H,I", [(160, 60000, 1024, 768), (40, 90000, 512, 384), (600, 30000, 256, 256)],
-                         ids=["g160", "g40", "g600_plain_wgrad_order"])
+TILE_TABLE_CASES = [(160, 60000, 1024, 768), (40, 90000, 512, 384), (600, 220000, 256, 256)]
+
+
+@pytest.mark.parametrize("G,A,H,I", TILE_TABLE_CASES, ids=["g160", "g40", "g600_plain_wgrad_order"])
 def test_tile_table_overflow_path(cuda, G, A, H, I):
     variant = build.variant_path("tiletab2")
     assert variant.exists(), f"{variant} is not built (python -m placemoe_amd.build)"
@@ -102,8 +107,10 @@ def test_tile_table_overflow_path(cuda, G, A, H, I):
         check_every_kind(cuda, off, H, I, 9, f"tiletab2 G={G}")
 
 
-@pytest.mark.parametrize("G,A,H,I", [(16, 20000, 1024, 512), (160, 30000, 512, 256), (5, 3000, 256, 192)],
-                         ids=["g16", "g160", "g5"])
+EIGHT_WAVE_CASES = [(16, 20000, 1024, 512), (160, 30000, 512, 256), (5, 3000, 256, 192), (600, 220000, 256, 192)]
+
+
+@pytest.mark.parametrize("G,A,H,I", EIGHT_WAVE_CASES, ids=["g16", "g160", "g5", "g600_plain_wgrad_order"])
 def test_eight_wave_build_every_kind(cuda, G, A, H, I):
     variant = build.variant_path("w8")
     assert variant.exists(), f"{variant} is not built (python -m placemoe_amd.build)"
