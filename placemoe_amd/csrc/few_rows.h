@@ -21,9 +21,10 @@ namespace fr {
 constexpr int kMaxG = 1024;  // groups (the m-tile prefix in LDS)
 
 // WM x WN waves, each FM x FN tiles of 16 x 16; NST stages; BPC blocks per CU.
-template <int WM_, int WN_, int FM_, int FN_, int KS_, int NST_, int BPC_>
+template <int WM_, int WN_, int FM_, int FN_, int NST_, int BPC_>
 struct Cfg {
-  static constexpr int WM = WM_, WN = WN_, FM = FM_, FN = FN_, KS = KS_, NST = NST_, BPC = BPC_;
+  static constexpr int WM = WM_, WN = WN_, FM = FM_, FN = FN_, NST = NST_, BPC = BPC_;
+  static constexpr int KS = 2;                     // k-steps (the MFMA's 32) of a K-tile
   static constexpr int KT = 32 * KS;               // depth of a K-tile
   static constexpr int CHK = KT / 8;               // 16-byte chunks of a K-contiguous row
   static constexpr int RPL = 64 / CHK;             // such rows per load
@@ -31,9 +32,9 @@ struct Cfg {
   static constexpr int BM = WM * FM * 16, BN = WN * FN * 16;
   static constexpr int A_BYTES = BM * KT * 2, B_BYTES = BN * KT * 2, STAGE = A_BYTES + B_BYTES;
   static constexpr int PA = A_BYTES / 1024, PB = B_BYTES / 1024;    // 1 KB loads per K-tile
-  static constexpr int QA = (PA + NW - 1) / NW, QB = PB / NW;       // ... of one wave
-  static_assert(PB % NW == 0 && (PA % NW == 0 || PA < NW), "whole loads per wave");
-  static_assert(KS == 2 && FN % 2 == 0 && NST >= 2 && (NST - 2) * (QA + QB) <= 63, "configuration");
+  static constexpr int QA = PA / NW, QB = PB / NW;                  // ... of one wave
+  static_assert(PB % NW == 0 && PA % NW == 0, "whole loads per wave");
+  static_assert(FN % 2 == 0 && NST >= 2 && (NST - 2) * (QA + QB) <= 63, "configuration");
 };
 
 // Operand loads of one wave for one output tile: the lane's byte offset of
@@ -47,13 +48,8 @@ struct Op {
   uint32_t kstep;  // offset per K-tile
 };
 
-// Chunk swizzle of K-contiguous rows: 16 consecutive rows read at one logical
-// chunk fall on 16 distinct 16-byte slots of the 256-byte bank line.
-template <class CF>
-__device__ __forceinline__ int swz(int row) { return CF::KS == 1 ? (row >> 2) & 3 : CF::KS == 2 ? kc_swz(row) : row & 15; }
-
 // K-contiguous operand rows (row, KT k): load q fills rows RPL*q .. +RPL-1,
-// lane i row RPL*q + i/CHK, physical chunk i%CHK = logical chunk ^ swz(row).
+// lane i row RPL*q + i/CHK, physical chunk i%CHK = logical chunk ^ kc_swz(row).
 // `src(row)` is the row's index in the operand, negative past its end.
 template <class CF, int Q, typename F>
 __device__ __forceinline__ void kc_setup(Op<Q>& op, int wave, int lane, int64_t ldb, int krem, F src) {
@@ -62,7 +58,7 @@ __device__ __forceinline__ void kc_setup(Op<Q>& op, int wave, int lane, int64_t 
 #pragma unroll
   for (int q0 = 0; q0 < Q; ++q0) {
     const int row = (q0 * CF::NW + wave) * CF::RPL + lane / CF::CHK;
-    const int c = (lane % CF::CHK) ^ swz<CF>(row);
+    const int c = (lane % CF::CHK) ^ kc_swz(row);
     const int64_t r = src(row);
     op.off[q0] = r >= 0 ? (uint32_t)(r * ldb) + (uint32_t)c * 16u : kOOB;
     op.tmask |= (c * 8 < krem ? 1u : 0u) << q0;
@@ -121,13 +117,12 @@ __device__ __forceinline__ void setup(const GemmParams& P, Tile<KIND, CF>& tc, i
 }
 
 // Load J of this wave's share of K-tile kt into `stage` (A: 0 .. QA-1, B: QA ..
-// QA+QB-1; a wave past a small A tile's last 1 KB piece issues only its QB).
+// QA+QB-1).
 template <int KIND, class CF, int J>
 __device__ __forceinline__ void issue(const GemmParams& P, char* stage, const Tile<KIND, CF>& tc, int32_t kt, int wave) {
   const bool tail = (int64_t)(kt + 1) * CF::KT > P.K;
   if constexpr (J < CF::QA) {
     const int q = J * CF::NW + wave;
-    if (CF::PA < CF::NW && q >= CF::PA) return;
     dma16(tc.A.r0, stage + q * 1024, tail && !((tc.A.tmask >> J) & 1u) ? kOOB : tc.A.off[J], (uint32_t)kt * tc.A.kstep);
   } else {
     constexpr int q0 = J - CF::QA;
@@ -369,7 +364,7 @@ __global__ __launch_bounds__(CF::NT, CF::NW * CF::BPC / 4) void few_rows_grouped
 #pragma unroll
   for (int ks = 0; ks < CF::KS; ++ks) {
     const int r = lane & 15;
-    sa[ks] = r * (CF::KT * 2) + (((ks * 4 + (lane >> 4)) ^ swz<CF>(r)) << 4);
+    sa[ks] = r * (CF::KT * 2) + (((ks * 4 + (lane >> 4)) ^ kc_swz(r)) << 4);
   }
   // fragments of [KT][BN] tiles: the lane's offset of each column block
   int32_t sb[CF::FN];
@@ -423,11 +418,10 @@ __global__ __launch_bounds__(CF::NT, CF::NW * CF::BPC / 4) void few_rows_grouped
     });
   };
   // The end of a K-tile: the next one has landed (at most the loads of the
-  // NST - 2 K-tiles issued after it are outstanding; a wave that skips its A
-  // load counts too few of them and waits for more), and every wave has read
+  // NST - 2 K-tiles issued after it are outstanding), and every wave has read
   // this one.
   auto turn = [&]() __attribute__((always_inline)) {
-    wait_loads_lds<(CF::NST - 2) * (CF::PA < NW ? CF::QB : L)>();
+    wait_loads_lds<(CF::NST - 2) * L>();
     block_barrier();
   };
 

@@ -2234,8 +2234,8 @@ constexpr bool use_w4() { return PMX_GEMM_W4 && ((PMX_W4_KINDS >> KIND) & 1); }
 #ifndef PMX_FEW_ROWS
 #define PMX_FEW_ROWS 1
 #endif
-using Few64 = fr::Cfg<1, 4, 4, 2, 2, 3, 2>;   // 64 x 128 tiles, 24 KB stages
-using Few128 = fr::Cfg<2, 4, 4, 4, 2, 3, 1>;  // 128 x 256 tiles, 48 KB stages
+using Few64 = fr::Cfg<1, 4, 4, 2, 3, 2>;   // 64 x 128 tiles, 24 KB stages
+using Few128 = fr::Cfg<2, 4, 4, 4, 3, 1>;  // 128 x 256 tiles, 48 KB stages
 // Weight gradients (us, fc2 + fc1; few-rows / four-wave kernel; 2048 x 768
 // unless stated): 160 copies of 5 rows 90 + 169 / 108 + 195, of 25 rows 85 +
 // 163 / 109 + 203, of 96 rows 102 + 215 / 128 + 240, 128 copies of 128 rows 100
