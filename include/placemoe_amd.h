@@ -75,8 +75,10 @@ int pmx_route(const int64_t* sel, const int64_t* M, const int64_t* src, int32_t 
 /* pmx_route that also stores the routing status word to `status_host` (NULL:
  * not stored): pinned host memory that the device can address, written by the
  * routing kernel at system scope.  A host that set the word to another value
- * beforehand can read from it, without waiting, whether the routing has run
- * and what it found.  The word must stay allocated until then. */
+ * beforehand can read from it, without waiting, whether the ids have been
+ * checked and what was found.  It says nothing of the outputs, which may still
+ * be in writing: they are ordered by the stream as usual.  The word must stay
+ * allocated until it has been written. */
 int pmx_route_reported(const int64_t* sel, const int64_t* M, const int64_t* src, int32_t src_const,
                        int32_t S, int32_t E, int64_t T, int32_t K, int32_t C,
                        int32_t* phys, int32_t* counts, int32_t* offsets, int32_t* pos,

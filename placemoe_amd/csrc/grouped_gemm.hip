@@ -2237,12 +2237,16 @@ constexpr bool use_w4() { return PMX_GEMM_W4 && ((PMX_W4_KINDS >> KIND) & 1); }
 using Few64 = fr::Cfg<1, 4, 4, 2, 3, 2>;   // 64 x 128 tiles, 24 KB stages
 using Few128 = fr::Cfg<2, 4, 4, 4, 3, 1>;  // 128 x 256 tiles, 48 KB stages
 // Weight gradients (us, fc2 + fc1; few-rows / four-wave kernel; 2048 x 768
-// unless stated): 160 copies of 5 rows 90 + 169 / 108 + 195, of 25 rows 85 +
-// 163 / 109 + 203, of 96 rows 102 + 215 / 128 + 240, 128 copies of 128 rows 100
-// + 200 / 113 + 208, of 256 rows 148 + 290 / 146 + 278; 32 copies of 60 rows of
-// 4096 x 1536 75 + 150 / 91 + 170.
-// The average says nothing of the hottest copies, whose K-tiles this kernel
-// loads one at a time: the line lies where even they have few.
+// unless stated): 160 copies of 5 rows 99 + 185 / 107 + 193, of 25 rows 86 +
+// 161 / 110 + 202, of 40 rows 90 + 180 / 116 + 210; 40 copies of 40 rows of
+// 2048 x 1416 48 + 85 / 99 + 107; 16 copies of 12 rows of 7168 x 2048 86 + 177 /
+// 99 + 177.  Over 22 layers 0.43 to 1.04 of the four-wave kernel's time from 4
+// rows per copy on; at 1-2 rows, where both mostly write zeros, up to 1.08 (one
+// gradient of a step; the step as a whole gains a third).  It still gains at 96
+// rows (95 + 193 / 111 + 197; Zipf(1.0) 93 + 177 / 137 + 224) and no longer at
+// 256 (153 + 309 / 155 + 299), but the average says nothing of the hottest
+// copies, whose K-tiles this kernel loads one at a time: the line lies where
+// even they have few.
 constexpr int64_t kFewRowsWgrad = 48;
 
 template <int KIND, class CF>
@@ -2299,7 +2303,8 @@ int launch(const GemmParams& P, hipStream_t stream) {
       if (tiling == Few128::BM) return launch_few<KIND, Few128>(P, grid, stream);
     }
     // FAST: K a multiple of 64, dgrad weights not split (P.b.split >= K).
-    // RS (register-staged operands): fc1 and fc2 always; the fc1 dgrad when
+    // RS (register-staged operands): fc2 always, fc1 where the four-wave kernel
+    // does not take it; the fc1 dgrad when
     // the copies are small (under 8 m-tiles of rows on average), where each
     // weight strip serves few tiles and its loads wait on memory - with a
     // few large copies the DMA path is faster (it spends less power).

@@ -270,7 +270,7 @@ __global__ __launch_bounds__(64) void route_rank_kernel(const int32_t* __restric
 // 16.8, 32768 37.6 / 16.5.
 constexpr int kSmallWaves = 16;
 constexpr int64_t kSmallMaxAssign = 8192;
-constexpr int kSmallMaxSlots = 896;  // (16 + 1) x C counters in 64 KB of LDS
+constexpr int kSmallMaxSlots = 896;  // 16 x C counters: 56 KB of LDS; one thread per copy in the scan
 
 __global__ __launch_bounds__(64 * kSmallWaves) void route_small_kernel(
     const int64_t* __restrict__ sel, const int64_t* __restrict__ M, const int64_t* __restrict__ src,

@@ -42,7 +42,7 @@ _PENDING_CHECKS: list = []
 
 def _sync_route_checks() -> bool:
     """PLACEMOE_AMD_CHECK_ROUTES=1: check every forward's routing on the spot
-    (one stream synchronisation per call)."""
+    (one wait for the routing's status per call)."""
     return os.environ.get("PLACEMOE_AMD_CHECK_ROUTES", "0") not in ("", "0")
 
 
